@@ -885,12 +885,7 @@ extern "C" int tah_quantile_stats_dev(tah_dev *dev, const float *q_dev, int32_t 
     return guarded(dev, [&] {
         check_quantiles(rows, n, alphas, n_alphas);
         if (rows == 0) return TAH_OK;
-        Loans loans(dev);
-        float *ad = loans.take<float>(std::max(n_alphas, 1));
-        if (n_alphas)
-            TAH_HIP(hipMemcpyAsync(ad, alphas, sizeof(float) * n_alphas, hipMemcpyHostToDevice, dev->stream));
-        quantile_stats(dev->stream, rows, n, q_dev, n_alphas, ad, stats_dev);
-        // the alphas' staging buffer goes back to the pool only once the copy from the caller's memory is done
+        quantile_stats(dev->stream, rows, n, q_dev, n_alphas, alphas, stats_dev);
         TAH_HIP(hipStreamSynchronize(dev->stream));
         return TAH_OK;
     });
@@ -904,11 +899,9 @@ extern "C" int tah_quantile_stats(tah_dev *dev, const float *q, int32_t rows, in
         if (rows == 0) return TAH_OK;
         Loans loans(dev);
         const size_t nin = (size_t)rows * n, nout = (size_t)rows * (3 + n_alphas);
-        float *qd = loans.take<float>(nin), *sd = loans.take<float>(nout), *ad = loans.take<float>(std::max(n_alphas, 1));
+        float *qd = loans.take<float>(nin), *sd = loans.take<float>(nout);
         TAH_HIP(hipMemcpyAsync(qd, q, sizeof(float) * nin, hipMemcpyHostToDevice, dev->stream));
-        if (n_alphas)
-            TAH_HIP(hipMemcpyAsync(ad, alphas, sizeof(float) * n_alphas, hipMemcpyHostToDevice, dev->stream));
-        quantile_stats(dev->stream, rows, n, qd, n_alphas, ad, sd);
+        quantile_stats(dev->stream, rows, n, qd, n_alphas, alphas, sd);
         TAH_HIP(hipMemcpyAsync(stats, sd, sizeof(float) * nout, hipMemcpyDeviceToHost, dev->stream));
         TAH_HIP(hipStreamSynchronize(dev->stream));
         return TAH_OK;
