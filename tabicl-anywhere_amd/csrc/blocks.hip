@@ -40,11 +40,12 @@ __device__ __forceinline__ void dma_to_lds(const uint8_t *src, uint8_t *dst, int
 
 constexpr int FFW = 4;  // wavefronts (of 32 rows each) per k_ff128 workgroup (eight, one workgroup a CU, measured slower)
 
-// The feed-forward body's start, by all 256 threads of a workgroup: the first weight slice's copy into slab (two
+// The feed-forward body's start, by all THREADS threads of a workgroup: the first weight slice's copy into slab (two
 // slices, 64 KB of LDS) and the first layer's bias into bias1 (256 floats of LDS).
+template <int THREADS = 64 * FFW>
 __device__ __forceinline__ void ff128_start(uint8_t *slab, float *bias1, const uint8_t *__restrict__ w1img,
                                             const float *__restrict__ b1, int tid) {
-    dma_to_lds<64 * FFW>(w1img, slab, SLAB, tid);
+    dma_to_lds<THREADS>(w1img, slab, SLAB, tid);
     if (tid < 64) reinterpret_cast<float4 *>(bias1)[tid] = reinterpret_cast<const float4 *>(b1)[tid];
 }
 
@@ -103,11 +104,11 @@ struct KvNext {
     float *out;
 };
 
-// x += l2(gelu(l1(norm2 x))) + b2 for 32 rows a wavefront (after ff128_start, all 256 threads): xv holds this lane's
+// x += l2(gelu(l1(norm2 x))) + b2 for 32 rows a wavefront (after ff128_start, all THREADS threads): xv holds this lane's
 // half of its row (columns 16 ks + 8 g + t); xrow is the row's storage, which holds x (read back for the residual
 // add) and takes the result (not where !live or !keep). With KV the result goes on, still in registers, through kn's
 // normalisation and projection (its four weight slices streamed after W2's) to kn.out (not where !live).
-template <bool KV = false>
+template <bool KV = false, int THREADS = 64 * FFW>
 __device__ __forceinline__ void ff128_rows(float (&xv)[8][8], bool live, float *xrow, uint8_t *slab, const float *bias1,
                                            const float *__restrict__ lnw, const float *__restrict__ lnb,
                                            const uint8_t *__restrict__ w1img, int s1,
@@ -137,7 +138,7 @@ __device__ __forceinline__ void ff128_rows(float (&xv)[8][8], bool live, float *
     auto next = [&](int j) {
         __builtin_amdgcn_s_waitcnt(0);  // this wavefront's copies of slice j have landed
         __syncthreads();                // everyone's have; slice j - 1's buffer is free
-        if (j + 1 < NSLICES) dma_to_lds<64 * FFW>(slice(j + 1), slab + ((j + 1) & 1) * SLAB, SLAB, tid);
+        if (j + 1 < NSLICES) dma_to_lds<THREADS>(slice(j + 1), slab + ((j + 1) & 1) * SLAB, SLAB, tid);
         return static_cast<const uint8_t *>(slab + (j & 1) * SLAB);
     };
     // acc[T] += (rows 32 T .. 32 T + 31 of the slice's weights) B over the slice's CPS 16-column steps
@@ -999,21 +1000,25 @@ __global__ __launch_bounds__(256, 2) void k_cell_block(int n, size_t sr, size_t 
 
 // ---- fused row block, attention half ------------------------------------------------------------------------------
 // x += out(attend(rope(Wq layer_norm1(x) + bq) / 4, rope(K), V)) + bo for every token of one row over all the row's
-// tokens (src/nn.rs:357-419, Rope src/nn.rs:304-321), for e = 128, 8 heads of 16 and T <= 128 tokens; the keys and
+// tokens (src/nn.rs:357-419, Rope src/nn.rs:304-321), for e = 128, 8 heads of 16 and T <= 32 W tokens; the keys and
 // values [T][2 e] (k then v per token, without rotation) come from a projection before it.
-// grid n rows; 256 threads; wavefront w owns tokens 32 w + 0..31 of row blockIdx.x, lane l token l % 32, as the B
+// grid n rows; W = 4 or 8 wavefronts; wavefront w owns tokens 32 w + 0..31 of row blockIdx.x, lane l token l % 32, as the B
 // operand of every product (as in k_cell_block):
 //  * the query projection as in k_cell_block, its accumulators rotated in registers (a coordinate's partner for the
 //    rotation sits on lane l ^ 32) and scaled by 1 / sqrt(16);
 //  * per head the workgroup stages the row's keys (rotated) and values into LDS split into fp16 halves, scaled by the
-//    head's power of two (one wavefront-pair's maximum each, across wavefronts through LDS): threads 0..127 a key
-//    each, threads 128..255 a value each, for the next head while the current one is attended (two barriers a head);
+//    head's power of two (one wavefront-pair's maximum each, across wavefronts through LDS): the first half of the threads a key
+//    each, the second a value each, for the next head while the current one is attended (two barriers a head);
 //  * keys past T are masked; the attention and the output projection then run as in k_cell_block.
 // With FF the block's feed-forward half follows in the same kernel, as in k_cell_block; with KV as well the next
 // row block's keys and values (kn.out [n][T][2 e], which may be kv itself: a workgroup reads only its own row's keys
 // and values, all of them before its feed-forward half starts).
-template <bool FF, bool KV>
-__global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *tok, const float *kv,
+//
+// W = 8 takes rows of 129 to 256 tokens, one workgroup a compute unit (two wavefronts a SIMD, as two workgroups of W =
+// 4). Bound by vector work as at W = 4. 500 rows of 204 tokens with KV: 264 us a launch, where the projection,
+// the rotation, the f32-MFMA attention, the output projection and the feed-forward apart took 480.
+template <bool FF, bool KV, int W>
+__global__ __launch_bounds__(64 * W, 2) void k_row_block(int T, int keep, float *tok, const float *kv,
                                                        const float *__restrict__ cosv, const float *__restrict__ sinv,
                                                        const float *__restrict__ n1w, const float *__restrict__ n1b,
                                                        const uint8_t *__restrict__ qimg, int qshift,
@@ -1023,13 +1028,15 @@ __global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *to
                                                        int s1, const uint8_t *__restrict__ w2img,
                                                        const float *__restrict__ b2, int s2, KvNext kn) {
     static_assert(FF || !KV, "the next block's keys and values come from the feed-forward's registers");
-    constexpr int E = 128;
-    __shared__ __align__(16) uint8_t lds[65536];
+    static_assert(W == 4 || W == 8, "the copies deal 8 KB over the threads");
+    constexpr int E = 128, THREADS = 64 * W, NT = 32 * W;  // NT: token slots
+    constexpr int STAGED = NT * 128;                       // a staged head: keys and values, hi and lo
+    __shared__ __align__(16) uint8_t lds[65536 < 32768 + 2 * STAGED ? 32768 + 2 * STAGED : 65536];
     __shared__ __align__(16) float ffb[FF ? 256 : 4];  // FF: the first feed-forward layer's bias
     __shared__ __align__(16) uint8_t zero[16], ones[16];
     __shared__ __align__(16) float qbs[128];
-    __shared__ __align__(16) float cst[2][128][8];  // cos, sin of token t, pair k
-    __shared__ float red[2][2][2];                  // [head parity][keys, values][wavefront of the pair]
+    __shared__ __align__(16) float cst[2][NT][8];  // cos, sin of token t, pair k
+    __shared__ float red[2][2][W / 2];              // [head parity][keys, values][wavefront of the half]
     __shared__ int shs[2][2];                       // [buffer][keys, values]: the staged head's scales
     uint8_t *const wo = lds;
     uint8_t *const kvl = lds + 32768;
@@ -1040,7 +1047,7 @@ __global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *to
     const bool live = tk < T;
     float *xrow = tok + ((size_t)row * T + (live ? tk : 0)) * E;
     const float *kvrow = kv + (size_t)row * T * 2 * E;
-    dma_to_lds(qimg, lds, 65536, tid);
+    dma_to_lds<THREADS>(qimg, lds, 65536, tid);
     if (tid < 4) reinterpret_cast<uint32_t *>(zero)[tid] = 0u;
     else if (tid < 8) reinterpret_cast<uint32_t *>(ones)[tid - 4] = 0x3c003c00u;
     if (tid < 32) reinterpret_cast<float4 *>(qbs)[tid] = *reinterpret_cast<const float4 *>(qb + 4 * tid);
@@ -1052,9 +1059,9 @@ __global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *to
         }
     }
 
-    // staging of head h: thread t < 128 takes key t (16 coordinates, rotated), thread 128 + t value t
-    const int st_tok = tid & 127;
-    const bool st_key = tid < 128, st_live = st_tok < T;
+    // staging of head h: thread t < NT takes key t (16 coordinates, rotated), thread NT + t value t
+    const int st_tok = tid & (NT - 1);
+    const bool st_key = tid < NT, st_live = st_tok < T;
     float stv[16];
     auto stage_load = [&](int h, int par) {
 #pragma unroll
@@ -1067,16 +1074,19 @@ __global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *to
 #pragma unroll
         for (int c = 0; c < 16; c++) mx = fmaxf(mx, fabsf(stv[c]));
         mx = wave_max(mx);
-        if (lane == 0) red[par][wave >> 1][wave & 1] = mx;
+        if (lane == 0) red[par][wave / (W / 2)][wave & (W / 2 - 1)] = mx;
     };
     auto stage_store = [&](int par) {
         // the keys' maximum is over the unrotated values: rotation keeps each pair's norm, so the rotated values stay
         // within sqrt(2) of it, and the split's scale (a maximum below 2^14) leaves that room
-        const int s = shift_for_max(fmaxf(red[par][st_key ? 0 : 1][0], red[par][st_key ? 0 : 1][1]) * 1.5f);
+        float mx = red[par][st_key ? 0 : 1][0];
+#pragma unroll
+        for (int i = 1; i < W / 2; i++) mx = fmaxf(mx, red[par][st_key ? 0 : 1][i]);
+        const int s = shift_for_max(mx * 1.5f);
         const float f = ldexpf(1.0f, s);
         if (st_tok == 0) shs[par][st_key ? 0 : 1] = s;
-        _Float16 *Kh = reinterpret_cast<_Float16 *>(kvl + par * 16384), *Kl = Kh + 2 * 128 * 8;
-        _Float16 *Vh = Kl + 2 * 128 * 8, *Vl = Vh + 8 * 2 * 16 * 8;
+        _Float16 *Kh = reinterpret_cast<_Float16 *>(kvl + par * STAGED), *Kl = Kh + 2 * NT * 8;
+        _Float16 *Vh = Kl + 2 * NT * 8, *Vl = Vh + NT / 16 * 2 * 16 * 8;
         if (st_key) {
             float rk[16];
 #pragma unroll
@@ -1090,8 +1100,8 @@ __global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *to
             split8(rk + 8, f, h1, l1);
             *reinterpret_cast<halfx8 *>(Kh + st_tok * 8) = h0;
             *reinterpret_cast<halfx8 *>(Kl + st_tok * 8) = l0;
-            *reinterpret_cast<halfx8 *>(Kh + (128 + st_tok) * 8) = h1;
-            *reinterpret_cast<halfx8 *>(Kl + (128 + st_tok) * 8) = l1;
+            *reinterpret_cast<halfx8 *>(Kh + (NT + st_tok) * 8) = h1;
+            *reinterpret_cast<halfx8 *>(Kl + (NT + st_tok) * 8) = l1;
         } else {
             const int st = st_tok >> 4, kg = (st_tok >> 3) & 1, t8 = st_tok & 7;
             const int sw = (2 * st + kg) & 15;
@@ -1205,7 +1215,7 @@ __global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *to
         for (int T4 = 0; T4 < 4; T4++) asm volatile("" : "+v"(qa[T4]));
     }
     __syncthreads();  // everyone is done with the query weights
-    dma_to_lds(oimg, wo, 32768, tid);
+    dma_to_lds<THREADS>(oimg, wo, 32768, tid);
     stage_store(0);
     stage_load(1, 1);
 
@@ -1221,7 +1231,7 @@ __global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *to
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();  // head h's keys and values are staged, head h + 1's maxima are in red; step h of the output
                           // weights has landed; everyone is done with head h - 1 and its buffer
-        if (h >= 1 && h + 3 < 8) dma_to_lds(oimg + (size_t)(h + 3) * 8192, wo + ((h + 3) & 3) * 8192, 8192, tid);
+        if (h >= 1 && h + 3 < 8) dma_to_lds<THREADS>(oimg + (size_t)(h + 3) * 8192, wo + ((h + 3) & 3) * 8192, 8192, tid);
         // one head ahead: head h + 1 into the buffer head h - 1 used, then head h + 2's values into registers
         if (h + 1 < 8) stage_store(par ^ 1);
         if (h + 2 < 8) stage_load(h + 2, par);
@@ -1229,8 +1239,8 @@ __global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *to
         int hl = lane;
         asm volatile("" : "+v"(hl));
         const int r32h = hl & 31, gh = hl >> 5, krow = sigma32(r32h), arow = krow;
-        const _Float16 *Kh = reinterpret_cast<const _Float16 *>(kvl + par * 16384), *Kl = Kh + 2 * 128 * 8;
-        const _Float16 *Vh = Kl + 2 * 128 * 8, *Vl = Vh + 8 * 2 * 16 * 8;
+        const _Float16 *Kh = reinterpret_cast<const _Float16 *>(kvl + par * STAGED), *Kl = Kh + 2 * NT * 8;
+        const _Float16 *Vh = Kl + 2 * NT * 8, *Vl = Vh + NT / 16 * 2 * 16 * 8;
         // this head's query coordinates: tile 0 holds heads h and h + 1 of an even h (the tiles shift down by one
         // after every second head, so that no register is indexed by the head)
         float qv[8];
@@ -1249,7 +1259,8 @@ __global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *to
 #pragma unroll
         for (int v = 0; v < 16; v++) o[v] = 0.0f;
 #pragma unroll
-        for (int k2 = 0; k2 < 2; k2++) {
+        for (int k2 = 0; k2 < NT / 64; k2++) {
+            if (k2 >= 2 && 64 * k2 >= T) continue;  // keys all past the row's tokens
             floatx16 sc[2];
             float mx = -INFINITY;
 #pragma unroll
@@ -1257,8 +1268,8 @@ __global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *to
 #pragma unroll
                 for (int v = 0; v < 16; v++) sc[j][v] = 0.0f;
                 const int key = 64 * k2 + 32 * j + krow;
-                const halfx8 ah = *reinterpret_cast<const halfx8 *>(Kh + (gh * 128 + key) * 8);
-                const halfx8 al = *reinterpret_cast<const halfx8 *>(Kl + (gh * 128 + key) * 8);
+                const halfx8 ah = *reinterpret_cast<const halfx8 *>(Kh + (gh * NT + key) * 8);
+                const halfx8 al = *reinterpret_cast<const halfx8 *>(Kl + (gh * NT + key) * 8);
                 sc[j] = mfma16x3(ah, al, qh, ql, sc[j]);
                 // accumulator v holds key 64 k2 + 32 j + 16 (v / 8) + 8 g + v % 8
                 const int lim = T - (64 * k2 + 32 * j) - 8 * gh;
@@ -1351,29 +1362,46 @@ __global__ __launch_bounds__(256, 2) void k_row_block(int T, int keep, float *to
         }
     if constexpr (FF) {
         __syncthreads();  // every wavefront is done with the attention's LDS (no copy is in flight after head 7)
-        ff128_start(lds, ffb, w1img, b1, tid);
+        ff128_start<THREADS>(lds, ffb, w1img, b1, tid);
         if constexpr (KV) {
             kn.out += ((size_t)row * T + (live ? tk : 0)) * 2 * E;
-            ff128_rows<true>(xn, live, xrow, lds, ffb, n2w, n2b, w1img, s1, w2img, b2, s2, tid, kn, tk < keep);
+            ff128_rows<true, THREADS>(xn, live, xrow, lds, ffb, n2w, n2b, w1img, s1, w2img, b2, s2, tid, kn, tk < keep);
         } else {
-            ff128_rows(xn, live, xrow, lds, ffb, n2w, n2b, w1img, s1, w2img, b2, s2, tid);
+            ff128_rows<false, THREADS>(xn, live, xrow, lds, ffb, n2w, n2b, w1img, s1, w2img, b2, s2, tid);
         }
     }
 }
 
 bool row_block_fits(const DevBlock &b, int T) {
-    return b.d == 128 && b.heads == 8 && b.inimg && b.outimg && T >= 1 && T <= 128;
+    return b.d == 128 && b.heads == 8 && b.inimg && b.outimg && T >= 1 && T <= 256;
 }
 
 bool block_ff_fits(const DevBlock &b) { return ff_fused_shape(b.d, b.ff) && b.l1img && b.l2img; }
 
 bool row_kv_fits(const DevBlock &next) { return next.d == 128 && next.inimg && next.in_b && next.n1w && next.n1b; }
 
+template <int W>
+static void launch_row_block(hipStream_t s, int n, int T, float *tok, const float *kv, const float *cosv, const float *sinv,
+                             const DevBlock &b, bool ff, bool next, const KvNext &kn, int keep) {
+    if (next)
+        hipLaunchKernelGGL((k_row_block<true, true, W>), dim3(n), dim3(64 * W), 0, s, T, keep, tok, kv, cosv, sinv, b.n1w,
+                           b.n1b, b.inimg, b.ins, b.in_b, b.outimg, b.outs, b.out_b, b.n2w, b.n2b, b.l1img, b.l1b, b.l1s,
+                           b.l2img, b.l2b, b.l2s, kn);
+    else if (ff)
+        hipLaunchKernelGGL((k_row_block<true, false, W>), dim3(n), dim3(64 * W), 0, s, T, T, tok, kv, cosv, sinv, b.n1w,
+                           b.n1b, b.inimg, b.ins, b.in_b, b.outimg, b.outs, b.out_b, b.n2w, b.n2b, b.l1img, b.l1b, b.l1s,
+                           b.l2img, b.l2b, b.l2s, KvNext{});
+    else
+        hipLaunchKernelGGL((k_row_block<false, false, W>), dim3(n), dim3(64 * W), 0, s, T, T, tok, kv, cosv, sinv, b.n1w,
+                           b.n1b, b.inimg, b.ins, b.in_b, b.outimg, b.outs, b.out_b, nullptr, nullptr, nullptr,
+                           nullptr, 0, nullptr, nullptr, 0, KvNext{});
+}
+
 void row_block(hipStream_t s, int n, int T, float *tok, const float *kv, const float *cosv, const float *sinv,
                const DevBlock &b, bool ff, const DevBlock *next, float *kv_next, int keep) {
     if (n <= 0) return;
     if (!row_block_fits(b, T) || (reinterpret_cast<uintptr_t>(tok) & 15) || (reinterpret_cast<uintptr_t>(kv) & 15))
-        throw ArgError{"row_block: needs e = 128, 8 heads, weight images, at most 128 tokens and aligned rows"};
+        throw ArgError{"row_block: needs e = 128, 8 heads, weight images, at most 256 tokens and aligned rows"};
     if (ff && !block_ff_fits(b)) throw ArgError{"row_block: no fused feed-forward weights for this shape"};
     if (next && (!ff || !row_kv_fits(*next) || !kv_next || (reinterpret_cast<uintptr_t>(kv_next) & 15)))
         throw ArgError{"row_block: the next block's keys and values need the fused feed-forward, e = 128, its "
@@ -1381,21 +1409,12 @@ void row_block(hipStream_t s, int n, int T, float *tok, const float *kv, const f
     if (keep < 0) keep = T;
     if (keep > T || (keep < T && !next))
         throw ArgError{"row_block: only a block that forms the next one's keys and values may leave tokens unwritten"};
-    if (next) {
-        const KvNext kn{next->inimg + (size_t)128 * 128 * 4, next->ins, next->n1w, next->n1b, next->in_b + 128,
-                        kv_next};
-        hipLaunchKernelGGL((k_row_block<true, true>), dim3(n), dim3(256), 0, s, T, keep, tok, kv, cosv, sinv, b.n1w, b.n1b,
-                           b.inimg, b.ins, b.in_b, b.outimg, b.outs, b.out_b, b.n2w, b.n2b, b.l1img, b.l1b, b.l1s,
-                           b.l2img, b.l2b, b.l2s, kn);
-    } else if (ff) {
-        hipLaunchKernelGGL((k_row_block<true, false>), dim3(n), dim3(256), 0, s, T, T, tok, kv, cosv, sinv, b.n1w, b.n1b,
-                           b.inimg, b.ins, b.in_b, b.outimg, b.outs, b.out_b, b.n2w, b.n2b, b.l1img, b.l1b, b.l1s,
-                           b.l2img, b.l2b, b.l2s, KvNext{});
-    } else {
-        hipLaunchKernelGGL((k_row_block<false, false>), dim3(n), dim3(256), 0, s, T, T, tok, kv, cosv, sinv, b.n1w,
-                           b.n1b, b.inimg, b.ins, b.in_b, b.outimg, b.outs, b.out_b, nullptr, nullptr, nullptr,
-                           nullptr, 0, nullptr, nullptr, 0, KvNext{});
-    }
+    const KvNext kn = next ? KvNext{next->inimg + (size_t)128 * 128 * 4, next->ins, next->n1w, next->n1b,
+                                    next->in_b + 128, kv_next}
+                           : KvNext{};
+    // a row's tokens as 32-token wavefronts, four or eight: the fewer the less work for slots past the row
+    if (T <= 128) launch_row_block<4>(s, n, T, tok, kv, cosv, sinv, b, ff, next != nullptr, kn, keep);
+    else launch_row_block<8>(s, n, T, tok, kv, cosv, sinv, b, ff, next != nullptr, kn, keep);
     TAH_LAUNCHED();
 }
 

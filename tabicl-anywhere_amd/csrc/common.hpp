@@ -205,7 +205,7 @@ void ff_block(hipStream_t s, int M, float *x, const DevBlock &b);
 // work: cell_block_work_bytes(groups) bytes, 16-byte aligned (the groups' key/value images).
 bool cell_block_fits(const DevBlock &b);
 // The attention half of a row block for every token of n rows of T tokens (tok [n][T][e] in place), from the keys
-// and values kv [n][T][2 e] the projection made (unrotated); e = 128, 8 heads of 16, T <= 128 (row_block_fits).
+// and values kv [n][T][2 e] the projection made (unrotated); e = 128, 8 heads of 16, T <= 256 (row_block_fits).
 // With ff (block_ff_fits) either kernel runs the block's feed-forward half as well, in the same launch; the row
 // block with next as well (ff, row_kv_fits) forms that block's keys and values [n][T][2 e] from the result into
 // kv_next (which may be kv), and then stores only the first keep tokens of each row's new values (the rest are

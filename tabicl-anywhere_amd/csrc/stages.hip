@@ -427,94 +427,29 @@ __global__ __launch_bounds__(256) void k_rope(size_t rows, int T, int e, int hea
     kh[k + half] = kb * c + ka * s;
 }
 
-// ---- attention within each row: head width 16, up to 16 * NT tokens -------------------------------------------
-// grid (rows, heads); 256 threads. Queries are the first nq_tok tokens of each row; out is [n][nq_tok][e].
-template <int NT>
-__global__ __launch_bounds__(256) void k_row_attn16(int n, int T, int nq_tok, int e, const float *__restrict__ qkv,
-                                                     float *__restrict__ out) {
-    constexpr int KT = 16 * NT;
-    __shared__ float Ks[16][KT + 4];
-    __shared__ float Vs[16][KT + 4];
-    const int r = blockIdx.x, h = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g4 = lane >> 4;
-    const float *base = qkv + (size_t)r * T * 3 * e;
-    for (int i = tid; i < 16 * KT; i += 256) {
-        const int k = i >> 4, c = i & 15;
-        const bool ok = k < T;
-        Ks[c][k] = ok ? base[(size_t)k * 3 * e + e + h * 16 + c] : 0.0f;
-        Vs[c][k] = ok ? base[(size_t)k * 3 * e + 2 * e + h * 16 + c] : 0.0f;
-    }
-    __syncthreads();
-    for (int qt = wave; qt * 16 < nq_tok; qt += 4) {
-        const int t = qt * 16 + r16;
-        const bool live = t < nq_tok;
-        float4 qv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (live) qv = *reinterpret_cast<const float4 *>(base + (size_t)t * 3 * e + h * 16 + 4 * g4);
-        const float qa[4] = {qv.x, qv.y, qv.z, qv.w};
-        floatx4 sacc[NT];
-#pragma unroll
-        for (int kt = 0; kt < NT; kt++) {
-            sacc[kt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int s = 0; s < 4; s++) sacc[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ks[4 * g4 + s][16 * kt + r16], qa[s], sacc[kt], 0, 0, 0);
-        }
-        float mx = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < NT; kt++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                if (16 * kt + 4 * g4 + v >= T) sacc[kt][v] = -INFINITY;
-                mx = fmaxf(mx, sacc[kt][v]);
-            }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        float l = 0.0f;
-#pragma unroll
-        for (int kt = 0; kt < NT; kt++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                sacc[kt][v] = fast_exp(sacc[kt][v] - mx);
-                l += sacc[kt][v];
-            }
-        l += __shfl_xor(l, 16, 64);
-        l += __shfl_xor(l, 32, 64);
-        floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int kt = 0; kt < NT; kt++) {
-            const float4 vv = *reinterpret_cast<const float4 *>(&Vs[r16][16 * kt + 4 * g4]);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.x, sacc[kt][0], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.y, sacc[kt][1], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.z, sacc[kt][2], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.w, sacc[kt][3], acc, 0, 0, 0);
-        }
-        if (live) {
-            const float inv = 1.0f / l;
-            *reinterpret_cast<float4 *>(out + ((size_t)r * nq_tok + t) * e + h * 16 + 4 * g4) =
-                make_float4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
-        }
-    }
-}
-
-// ---- the class tokens' attention within each row: head width 16, at most 4 queries, T <= 128 ----------------------
-// grid n rows; 64 x heads threads (at most 8 heads), wavefront h head h. Few queries against at most 128 keys: plain f32 arithmetic,
-// each row's keys and values read once by its workgroup (the heads' slices of a token side by side). Lane l takes
-// tokens l and l + 64: their keys (rotated, the k_rope formula) and values, the scores of the (rotated, 1 / sqrt(16))
+// ---- the class tokens' attention within each row: head width 16, at most 4 queries, T <= 64 J ---------------------
+// grid (n rows, heads / H); 64 x H threads (at most 8 heads), a wavefront a head. Few queries against the row's keys: plain
+// f32 arithmetic, each row's keys and values read once (the heads' slices of a token side by side). Rows of more than
+// 128 tokens take J = 4 with H = 4 heads a workgroup, whose LDS then still holds two workgroups a compute unit. Lane l
+// takes tokens l + 64 j: their keys (rotated, the k_rope formula) and values, the scores of the (rotated, 1 / sqrt(16))
 // queries, the softmax over the row's tokens by wavefront reductions; the weights and values then go through LDS,
 // and lane c = 16 i + j forms coordinate j of query i's output. Keys of token t of row r at kv + r * kv_row +
 // t * kv_tok (values e floats further), query i at q + r * q_row + i * q_tok.
 constexpr int CLS_MAXQ = 4;
-__global__ __launch_bounds__(512) void k_cls_attn(int n, int T, int nq, int e, const float *__restrict__ kv,
+template <int J, int H>
+__global__ __launch_bounds__(64 * H) void k_cls_attn(int n, int T, int nq, int e, const float *__restrict__ kv,
                                                    size_t kv_row, int kv_tok, const float *__restrict__ q, size_t q_row,
                                                    int q_tok, const float *__restrict__ cosv,
                                                    const float *__restrict__ sinv, float *__restrict__ out) {
-    __shared__ float ps[8][CLS_MAXQ][128];            // [head][query][token] weights
-    __shared__ __align__(16) float vs[8][128][16];    // [head][token][coordinate] values
-    const int r = blockIdx.x, h = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ float ps[H][CLS_MAXQ][64 * J];            // [head][query][token] weights
+    __shared__ __align__(16) float vs[H][64 * J][16];    // [head][token][coordinate] values
+    const int r = blockIdx.x, wave = threadIdx.x >> 6, h = blockIdx.y * H + wave, lane = threadIdx.x & 63;
+    if (h * 16 >= e) return;  // whole wavefronts leave together
     const float *kr = kv + (size_t)r * kv_row + h * 16;
-    float k2[2][16];
-    bool tl[2];
+    float k2[J][16];
+    bool tl[J];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
+    for (int j = 0; j < J; j++) {
         const int t = lane + 64 * j;
         tl[j] = t < T;
         const float *kp = kr + (size_t)(tl[j] ? t : 0) * kv_tok;
@@ -538,7 +473,7 @@ __global__ __launch_bounds__(512) void k_cls_attn(int n, int T, int nq, int e, c
         if (tl[j]) {
 #pragma unroll
             for (int c = 0; c < 16; c += 4)
-                *reinterpret_cast<float4 *>(&vs[h][t][c]) = make_float4(v16[c], v16[c + 1], v16[c + 2], v16[c + 3]);
+                *reinterpret_cast<float4 *>(&vs[wave][t][c]) = make_float4(v16[c], v16[c + 1], v16[c + 2], v16[c + 3]);
         }
     }
     float lsum[CLS_MAXQ];
@@ -558,20 +493,23 @@ __global__ __launch_bounds__(512) void k_cls_attn(int n, int T, int nq, int e, c
             qv[k] = (a * cs[k] - b * sn[k]) * 0.25f;
             qv[k + 8] = (b * cs[k] + a * sn[k]) * 0.25f;
         }
-        float sc[2];
+        float sc[J];
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
+        for (int j = 0; j < J; j++) {
             float a = 0.0f;
 #pragma unroll
             for (int c = 0; c < 16; c++) a += qv[c] * k2[j][c];
             sc[j] = tl[j] ? a : -INFINITY;
         }
-        const float mx = wave_max(fmaxf(sc[0], sc[1]));
+        float mx = sc[0];
+#pragma unroll
+        for (int j = 1; j < J; j++) mx = fmaxf(mx, sc[j]);
+        mx = wave_max(mx);
         float l = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
+        for (int j = 0; j < J; j++) {
             const float pj = tl[j] ? exp2_hw((sc[j] - mx) * LOG2E) : 0.0f;
-            ps[h][i][lane + 64 * j] = pj;
+            ps[wave][i][lane + 64 * j] = pj;
             l += pj;
         }
         lsum[i] = wave_sum(l);
@@ -581,7 +519,7 @@ __global__ __launch_bounds__(512) void k_cls_attn(int n, int T, int nq, int e, c
     const int qi = lane >> 4, c = lane & 15;
     if (qi >= nq) return;
     float o = 0.0f;
-    for (int t = 0; t < T; t++) o += ps[h][qi][t] * vs[h][t][c];
+    for (int t = 0; t < T; t++) o += ps[wave][qi][t] * vs[wave][t][c];
     float l = lsum[0];
 #pragma unroll
     for (int i = 1; i < CLS_MAXQ; i++)
@@ -589,27 +527,30 @@ __global__ __launch_bounds__(512) void k_cls_attn(int n, int T, int nq, int e, c
     out[((size_t)r * nq + qi) * e + h * 16 + c] = o / l;
 }
 
-// ---- attention within each row on split-fp16 MFMA, rotary positions folded in: head width 16, T <= 128 ---------
+// ---- attention within each row on split-fp16 MFMA, rotary positions folded in: head width 16, T <= 32 KT -------
 // grid (rows, heads); 256 threads. The row's keys and values of head h are loaded once per workgroup (one thread per
 // token), the keys rotated (RoPE, the k_rope formula), both scaled by the power of two that brings the head's
 // largest magnitude below 2^14 and split into fp16 hi/lo in LDS: K as [k half][key][8], V^T as
 // [16-key step][k half][coordinate][8] (every 16-lane read contiguous; coordinates XOR-swizzled by block so the
 // scattered writes spread over the banks). Wavefront w then takes query tokens
-// 32 w .. 32 w + 31 (lane = query, its two halves of the head's 16 coordinates on lanes l and l + 32, rotated
-// with one cross-lane exchange and multiplied by 1 / sqrt(16)): S^T = K Q^T for four 32-key tiles (K in sigma32
+// 32 w .. 32 w + 31, and 128 on (lane = query, its two halves of the head's 16 coordinates on lanes l and l + 32, rotated
+// with one cross-lane exchange and multiplied by 1 / sqrt(16)): S^T = K Q^T for KT 32-key tiles (K in sigma32
 // order), a plain softmax over the row's tokens (weights at most 2^12), and O^T = V^T P^T with the weights straight
 // from the accumulators as the B operand; V^T fills 16 of the 32 A-operand rows (the rest are zeros).
 // One dimension of n x heads workgroups: consecutive workgroups go to the eight XCDs in turn, and workgroup i takes
 // (row, head) number (i % 8) G / 8 + i / 8, heads fastest: an XCD runs a row's heads together, so its L2 reads the
 // row's keys and values once. Query token t of row r at q + r * q_row + t * q_tok (the projection's [T][3 e]
 // layout, or the class tokens' own [cls][e]).
+// KT = 8 takes rows of 129 to 256 tokens, a token a thread still, below 128 rows (64 rows of 204 tokens, a whole
+// prediction: 0.775 ms, 0.867 with the row block's kernel, whose 64 workgroups leave most compute units idle).
+template <int KT>
 __global__ __launch_bounds__(256) void k_row_attn_x3(int n, int T, int nq_tok, int e, int heads,
                                                       const float *__restrict__ qkv,
                                                       const float *__restrict__ q, size_t q_row, int q_tok,
                                                       const float *__restrict__ cosv, const float *__restrict__ sinv,
                                                       float *__restrict__ out) {
-    __shared__ __align__(16) _Float16 Kh[2][128][8], Kl[2][128][8];
-    __shared__ __align__(16) _Float16 Vh[8][2][16][8], Vl[8][2][16][8];
+    __shared__ __align__(16) _Float16 Kh[2][32 * KT][8], Kl[2][32 * KT][8];
+    __shared__ __align__(16) _Float16 Vh[2 * KT][2][16][8], Vl[2 * KT][2][16][8];
     __shared__ float red[2][4];
     const int G = gridDim.x;
     const int item = G % 8 == 0 ? (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3) : blockIdx.x;
@@ -656,7 +597,7 @@ __global__ __launch_bounds__(256) void k_row_attn_x3(int n, int T, int nq_tok, i
     __syncthreads();
     const int sk = shift_for_max(fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3])));
     const int sv = shift_for_max(fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3])));
-    if (tid < 128) {
+    if (tid < 32 * KT) {
         halfx8 h0, l0, h1, l1;
         split8(kv, ldexpf(1.0f, sk), h0, l0);
         split8(kv + 8, ldexpf(1.0f, sk), h1, l1);
@@ -678,100 +619,96 @@ __global__ __launch_bounds__(256) void k_row_attn_x3(int n, int T, int nq_tok, i
     }
     __syncthreads();
     const int r32 = lane & 31, g = lane >> 5;
-    const int qt = wave * 32 + r32;  // query token
-    if (wave * 32 >= nq_tok) return;
-    const bool live = qt < nq_tok;
-    // this lane's half of the query's coordinates (8 g .. 8 g + 7), rotated with the other half from lane l ^ 32
-    float qv[8];
-    {
-        float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
-        if (live) {
-            const float *qp = q + (size_t)r * q_row + (size_t)qt * q_tok + h * 16 + 8 * g;
-            a = *reinterpret_cast<const float4 *>(qp);
-            b = *reinterpret_cast<const float4 *>(qp + 4);
+    for (int q0 = wave * 32; q0 < nq_tok; q0 += 128) {
+        const int qt = q0 + r32;  // query token
+        const bool live = qt < nq_tok;
+        // this lane's half of the query's coordinates (8 g .. 8 g + 7), rotated with the other half from lane l ^ 32
+        float qv[8];
+        {
+            float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
+            if (live) {
+                const float *qp = q + (size_t)r * q_row + (size_t)qt * q_tok + h * 16 + 8 * g;
+                a = *reinterpret_cast<const float4 *>(qp);
+                b = *reinterpret_cast<const float4 *>(qp + 4);
+            }
+            qv[0] = a.x; qv[1] = a.y; qv[2] = a.z; qv[3] = a.w; qv[4] = b.x; qv[5] = b.y; qv[6] = b.z; qv[7] = b.w;
+            const float sgn = g == 0 ? -1.0f : 1.0f;
+            float cs[8] = {1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f}, sn[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+            if (live) {
+                load8(cosv + qt * 8, cs);
+                load8(sinv + qt * 8, sn);
+            }
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const float other = __shfl_xor(qv[k], 32, 64);
+                qv[k] = (qv[k] * cs[k] + sgn * other * sn[k]) * 0.25f;  // (a c - b s) or (b c + a s), times 1 / sqrt(16)
+            }
         }
-        qv[0] = a.x; qv[1] = a.y; qv[2] = a.z; qv[3] = a.w; qv[4] = b.x; qv[5] = b.y; qv[6] = b.z; qv[7] = b.w;
-        const float sgn = g == 0 ? -1.0f : 1.0f;
-        float cs[8] = {1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f}, sn[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        if (live) {
-            load8(cosv + qt * 8, cs);
-            load8(sinv + qt * 8, sn);
+        float qmax = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) qmax = fmaxf(qmax, fabsf(qv[k]));
+        qmax = fmaxf(qmax, __shfl_xor(qmax, 32, 64));
+        const int sq = shift_for_max(qmax);
+        halfx8 qh, ql;
+        split8(qv, ldexpf(1.0f, sq), qh, ql);
+        const float to_log2 = ldexpf(LOG2E, -(sk + sq));  // raw score -> score * log2 e (positive)
+        // S^T: key tiles of 32, rows in sigma32 order; accumulator v of tile kt holds key 32 kt + 16 (v / 8) + 8 g + v % 8
+        const int krow = sigma32(r32);
+        floatx16 sc[KT];
+        float mx = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) sc[kt][v] = 0.0f;
+            const int key = 32 * kt + krow;  // keys past T are zero rows, masked below
+            const halfx8 ah = *reinterpret_cast<const halfx8 *>(&Kh[g][key][0]);
+            const halfx8 al = *reinterpret_cast<const halfx8 *>(&Kl[g][key][0]);
+            sc[kt] = mfma16x3(ah, al, qh, ql, sc[kt]);
+            if (32 * kt + 32 > T) {
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    if (32 * kt + 16 * (v >> 3) + 8 * g + (v & 7) >= T) sc[kt][v] = -INFINITY;
+            }
+#pragma unroll
+            for (int v = 0; v < 16; v++) mx = fmaxf(mx, sc[kt][v]);
         }
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float off = 12.0f - mx * to_log2;
+        float l = 0.0f;
+        // O^T = V^T P^T over the 16-key steps st = 2 kt + hh: A rows 0..15 the coordinates, 16..31 zero
+        floatx16 o;
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const float other = __shfl_xor(qv[k], 32, 64);
-            qv[k] = (qv[k] * cs[k] + sgn * other * sn[k]) * 0.25f;  // (a c - b s) or (b c + a s), times 1 / sqrt(16)
-        }
-    }
-    float qmax = 0.0f;
+        for (int v = 0; v < 16; v++) o[v] = 0.0f;
+        halfx8 zero8;
 #pragma unroll
-    for (int k = 0; k < 8; k++) qmax = fmaxf(qmax, fabsf(qv[k]));
-    qmax = fmaxf(qmax, __shfl_xor(qmax, 32, 64));
-    const int sq = shift_for_max(qmax);
-    halfx8 qh, ql;
-    split8(qv, ldexpf(1.0f, sq), qh, ql);
-    const float to_log2 = ldexpf(LOG2E, -(sk + sq));  // raw score -> score * log2 e (positive)
-    // S^T: key tiles of 32, rows in sigma32 order; accumulator v of tile kt holds key 32 kt + 16 (v / 8) + 8 g + v % 8
-    const int krow = sigma32(r32);
-    floatx16 sc[4];
-    float mx = -INFINITY;
+        for (int t = 0; t < 8; t++) zero8[t] = (_Float16)0.0f;
 #pragma unroll
-    for (int kt = 0; kt < 4; kt++) {
-#pragma unroll
-        for (int v = 0; v < 16; v++) sc[kt][v] = 0.0f;
-        const int key = 32 * kt + krow;  // keys past T are zero rows, masked below
-        const halfx8 ah = *reinterpret_cast<const halfx8 *>(&Kh[g][key][0]);
-        const halfx8 al = *reinterpret_cast<const halfx8 *>(&Kl[g][key][0]);
-        sc[kt] = mfma16x3(ah, al, qh, ql, sc[kt]);
-        if (32 * kt + 32 > T) {
-#pragma unroll
-            for (int v = 0; v < 16; v++)
-                if (32 * kt + 16 * (v >> 3) + 8 * g + (v & 7) >= T) sc[kt][v] = -INFINITY;
-        }
-#pragma unroll
-        for (int v = 0; v < 16; v++) mx = fmaxf(mx, sc[kt][v]);
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float off = 12.0f - mx * to_log2;
-    float l = 0.0f;
-    halfx8 ph[8], pl[8];  // 16-key step s = 2 kt + hh
-#pragma unroll
-    for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-        for (int hh = 0; hh < 2; hh++) {
+        for (int st = 0; st < 2 * KT; st++) {
+            if (16 * st >= T) continue;  // weights 0
             float p[8];
 #pragma unroll
             for (int t = 0; t < 8; t++) {
-                p[t] = exp2_hw(fmaf(sc[kt][8 * hh + t], to_log2, off));
+                p[t] = exp2_hw(fmaf(sc[st >> 1][8 * (st & 1) + t], to_log2, off));
                 l += p[t];
             }
-            split8(p, 1.0f, ph[2 * kt + hh], pl[2 * kt + hh]);
+            halfx8 ph, pl;
+            split8(p, 1.0f, ph, pl);
+            halfx8 ah = zero8, al = zero8;
+            if (r32 < 16) {
+                const int row = r32 ^ ((2 * st + g) & 15);
+                ah = *reinterpret_cast<const halfx8 *>(&Vh[st][g][row][0]);
+                al = *reinterpret_cast<const halfx8 *>(&Vl[st][g][row][0]);
+            }
+            o = mfma16x3(ah, al, ph, pl, o);
         }
-    l += __shfl_xor(l, 32, 64);
-    // O^T = V^T P^T: A rows 0..15 the coordinates, 16..31 zero
-    floatx16 o;
-#pragma unroll
-    for (int v = 0; v < 16; v++) o[v] = 0.0f;
-    halfx8 zero8;
-#pragma unroll
-    for (int t = 0; t < 8; t++) zero8[t] = (_Float16)0.0f;
-#pragma unroll
-    for (int st = 0; st < 8; st++) {
-        if (16 * st >= T) break;
-        halfx8 ah = zero8, al = zero8;
-        if (r32 < 16) {
-            const int row = r32 ^ ((2 * st + g) & 15);
-            ah = *reinterpret_cast<const halfx8 *>(&Vh[st][g][row][0]);
-            al = *reinterpret_cast<const halfx8 *>(&Vl[st][g][row][0]);
-        }
-        o = mfma16x3(ah, al, ph[st], pl[st], o);
+        l += __shfl_xor(l, 32, 64);
+        if (!live) continue;
+        // accumulator v < 8 holds coordinate 8 (v / 4) + 4 g + v % 4 of this lane's query
+        const float f = ldexpf(1.0f, -sv) / l;
+        float *dst = out + ((size_t)r * nq_tok + qt) * e + h * 16;
+        *reinterpret_cast<float4 *>(dst + 4 * g) = make_float4(o[0] * f, o[1] * f, o[2] * f, o[3] * f);
+        *reinterpret_cast<float4 *>(dst + 8 + 4 * g) = make_float4(o[4] * f, o[5] * f, o[6] * f, o[7] * f);
     }
-    if (!live) return;
-    // accumulator v < 8 holds coordinate 8 (v / 4) + 4 g + v % 4 of this lane's query
-    const float f = ldexpf(1.0f, -sv) / l;
-    float *dst = out + ((size_t)r * nq_tok + qt) * e + h * 16;
-    *reinterpret_cast<float4 *>(dst + 4 * g) = make_float4(o[0] * f, o[1] * f, o[2] * f, o[3] * f);
-    *reinterpret_cast<float4 *>(dst + 8 + 4 * g) = make_float4(o[4] * f, o[5] * f, o[6] * f, o[7] * f);
 }
 
 // Any head width and token count: one thread per (row, query token, head).
@@ -894,7 +831,10 @@ constexpr int SMALL_ROWS = 2048;
 // projections, the attention (a workgroup per row and head) and the output projection separately (measured: one
 // row 0.84 -> 0.76 ms a prediction, 64 rows 1.43 -> 1.40 ms).
 constexpr int ROW_BLOCK_MIN = 128;
-constexpr int CLS_QUERIES_MIN = 512;
+// The last row block queries the class tokens alone from this many rows: 512 of up to 128 tokens, every row count that
+// the row block takes of more, whose other tokens' queries cost more (204 tokens, a prediction without and with: 140
+// rows 0.981 and 0.970 ms, 200 1.033 and 0.996, 500 1.656 and 1.591).
+static int cls_queries_min(int T) { return T <= 128 ? 512 : ROW_BLOCK_MIN; }
 
 // x [M][e] += l2(gelu(l1(norm2 x))): the fused kernel where the block's shape has one (above SMALL_ROWS rows), else
 // two GEMMs with the norm folded into the first where it fits, else layer_norm and two GEMMs (t [M][e] and mid [M][ff]
@@ -1105,10 +1045,10 @@ void class_token_kv(hipStream_t s, const tah_weights *w, float *out, float *tmp)
 }
 
 
-// The row stage's fused kernels: head width 16 with the rotary tables' 8 frequencies, at most 128 tokens (the
+// The row stage's fused kernels: head width 16 with the rotary tables' 8 frequencies, at most 256 tokens (the
 // rotary positions applied inside the attention kernels).
 static bool row_fused(const tah_weights *w, int T) {
-    return w->row_heads > 0 && w->e / w->row_heads == 16 && w->e % w->row_heads == 0 && w->rope_half == 8 && T <= 128;
+    return w->row_heads > 0 && w->e / w->row_heads == 16 && w->e % w->row_heads == 0 && w->rope_half == 8 && T <= 256;
 }
 
 // Whether row block bi runs as k_row_block (one kernel, a workgroup per row) for n rows of T tokens.
@@ -1130,7 +1070,7 @@ static bool row_stage_compact(const tah_weights *w, int n, int T) {
     const size_t R = (size_t)n * T;
     for (int bi = 0; bi < last; bi++)
         if (!row_block_path(w, bi, n, T) || !block_ff_fits(w->row[bi]) || R <= SMALL_ROWS) return false;
-    return w->row[last].inimg && n >= CLS_QUERIES_MIN && w->cls <= CLS_MAXQ && w->row_heads <= 8;
+    return w->row[last].inimg && n >= cls_queries_min(T) && w->cls <= CLS_MAXQ && w->row_heads <= 8;
 }
 
 // The row stage's scratch, in floats; row_stage lays it out as:
@@ -1165,28 +1105,26 @@ void row_stage(hipStream_t s, const tah_weights *w, float *tok, int n, int T, co
     if (2 * half != hd) throw ArgError{"row stage: rotary frequencies must cover half the head width"};
     const float inv = 1.0f / sqrtf((float)hd);
     const int last = w->row_blocks - 1;
-    const bool mfma = hd == 16 && T <= 256;
     const bool fused = row_fused(w, T);  // rotary positions applied inside k_row_attn_x3
     // the queries k_row_attn_x3 reads: the projection's [T][3 e] rows, or (the last block) the class tokens' [cls][e]
     const float *q_of = qkv;
     size_t q_row = (size_t)T * 3 * e;
     int q_tok = 3 * e;
     auto attend = [&](int nq_tok, float *dst) {
-        if (fused)
-            hipLaunchKernelGGL(k_row_attn_x3, dim3(n * heads), dim3(256), 0, s, n, T, nq_tok, e, heads, qkv, q_of,
+        if (fused && T <= 128)
+            hipLaunchKernelGGL(k_row_attn_x3<4>, dim3(n * heads), dim3(256), 0, s, n, T, nq_tok, e, heads, qkv, q_of,
                                q_row, q_tok, cosv, sinv, dst);
-        else if (mfma && T <= 128)
-            hipLaunchKernelGGL(k_row_attn16<8>, dim3(n, heads), dim3(256), 0, s, n, T, nq_tok, e, qkv, dst);
-        else if (mfma)
-            hipLaunchKernelGGL(k_row_attn16<16>, dim3(n, heads), dim3(256), 0, s, n, T, nq_tok, e, qkv, dst);
+        else if (fused)
+            hipLaunchKernelGGL(k_row_attn_x3<8>, dim3(n * heads), dim3(256), 0, s, n, T, nq_tok, e, heads, qkv, q_of,
+                               q_row, q_tok, cosv, sinv, dst);
         else
             hipLaunchKernelGGL(k_row_attn_plain, blocks_for((size_t)n * nq_tok * heads), dim3(256), 0, s, n, T, nq_tok, e,
                                heads, qkv, dst);
         TAH_LAUNCHED();
     };
-    // the last block's path: only the class tokens queried (from CLS_QUERIES_MIN rows), by k_cls_attn where it
+    // the last block's path: only the class tokens queried (from cls_queries_min rows), by k_cls_attn where it
     // takes the shape
-    const bool cls_path = fused && w->row[last].inimg && n >= CLS_QUERIES_MIN;
+    const bool cls_path = fused && w->row[last].inimg && n >= cls_queries_min(T);
     const bool cls_kernel = cls_path && cls <= CLS_MAXQ && heads <= 8;
     // kv_ready: this block's keys and values are in qkv [R][2 e] already (formed by the block before it)
     for (int bi = 0; bi <= last; bi++) {
@@ -1213,7 +1151,7 @@ void row_stage(hipStream_t s, const tah_weights *w, float *tok, int n, int T, co
             // the last block queries only the class tokens: keys and values for every token (the projection's second
             // and third 128-row blocks: qkv [R][2 e] for k_cls_attn, unless the previous block formed them, else into
             // qkv's [T][3 e] rows), queries for the class tokens alone, from their gathered copy (which the block
-            // then updates); below CLS_QUERIES_MIN rows the extra launch costs more than the other tokens' queries
+            // then updates); below cls_queries_min rows the extra launch costs more than the other tokens' queries
             // (2,048 rows 4.30 -> 4.25 ms, 64 and 256 rows 5 us slower)
             if (!kv_ready)
                 rows128(s, (int)R, 2 * e, tok, e, b.inimg + (size_t)128 * e * 4, b.ins, b.in_b + e,
@@ -1224,8 +1162,12 @@ void row_stage(hipStream_t s, const tah_weights *w, float *tok, int n, int T, co
             TAH_LAUNCHED();
             rows128(s, M, e, xc, e, b.inimg, b.ins, b.in_b, ac, e, EPI_NONE, nullptr, 0, nullptr, b.n1w, b.n1b);
             if (cls_kernel) {
-                hipLaunchKernelGGL(k_cls_attn, dim3(n), dim3(64 * heads), 0, s, n, T, cls, e, qkv, (size_t)T * 2 * e,
-                                   2 * e, ac, (size_t)cls * e, e, cosv, sinv, att);
+                if (T <= 128)
+                    hipLaunchKernelGGL((k_cls_attn<2, 8>), dim3(n), dim3(64 * heads), 0, s, n, T, cls, e, qkv,
+                                       (size_t)T * 2 * e, 2 * e, ac, (size_t)cls * e, e, cosv, sinv, att);
+                else
+                    hipLaunchKernelGGL((k_cls_attn<4, 4>), dim3(n, (heads + 3) / 4), dim3(256), 0, s, n, T, cls, e, qkv,
+                                       (size_t)T * 2 * e, 2 * e, ac, (size_t)cls * e, e, cosv, sinv, att);
                 TAH_LAUNCHED();
             } else {
                 q_of = ac;
