@@ -8,16 +8,32 @@ namespace tah {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
+// v of lane i ^ 1, i ^ 2, then (quads being alike) of the other quad of eight lanes and the other eight of sixteen, by
+// DPP: no trip through the LDS crossbar, as a shuffle would take
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+
+// op over all 64 lanes, in every lane: in pairs of lanes 1, 2, 4, 8, 16 and 32 apart
+template <class F>
+__device__ __forceinline__ float wave_reduce(float v, F &&op) {
+    v = op(v, dpp<0xb1>(v));   // quad_perm [1, 0, 3, 2]
+    v = op(v, dpp<0x4e>(v));   // quad_perm [2, 3, 0, 1]
+    v = op(v, dpp<0x141>(v));  // row_half_mirror
+    v = op(v, dpp<0x140>(v));  // row_mirror
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return wave_reduce(v, [](float a, float b) { return a + b; });
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+    return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 constexpr float LOG2E = 1.44269504088896340736f;
