@@ -1640,12 +1640,6 @@ __global__ __launch_bounds__(256) void k_attn_merge_w(int items, int splits, con
     out[(size_t)i * 64 + lane] = O / L;
 }
 
-void merge_splits(hipStream_t s, int nq, int d, int heads, int splits, const float *part_o, const float *part_ml,
-                  float *out) {
-    hipLaunchKernelGGL(k_attn_merge, dim3(nq * heads), dim3(64), 0, s, nq, d, heads, splits, 0, part_o, part_ml, out);
-    TAH_LAUNCHED();
-}
-
 // ---- planning and launch --------------------------------------------------------------------------------------
 struct AttnPlan {
     bool split16, few;  // few: k_attn_few (any tiles, at most FEW_Q queries; i16 from FEW16_FROM)

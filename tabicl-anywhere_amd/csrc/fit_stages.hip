@@ -4,14 +4,14 @@
 //
 // Per batch of feature groups (cells [groups][rows][e], group-major so each group's cells are contiguous):
 // input layer and target embedding (per label digit), then per column block: the inducing points' queries attend
-// to the group's cells (k_ind_attn16: online softmax over key blocks of 64 cells, fp32 MFMA, split over key ranges
+// to the group's cells (k_ind_attn16: online softmax over blocks of 128 cells, split-fp16 MFMA, split over key ranges
 // and merged as in the in-context attention), the inducing points' output projection and feed-forward, their keys
 // and values for the second attention written straight into the column cache layout, and the cells' own block
 // against them (column_block, shared with prediction).
 #include <algorithm>
 
+#include "attend.hpp"
 #include "common.hpp"
-#include "device_math.hpp"
 
 namespace tah {
 
@@ -88,98 +88,168 @@ __global__ __launch_bounds__(256) void k_col_records(int gb, int inds, int e, co
     col_kv[(size_t)(g0 + gl) * gstride + off + (size_t)j * inds + k] = kv2[((size_t)gl * inds + k) * 2 * e + j];
 }
 
-// The inducing points' queries indq [inds][e] over one group's cells, keys and values from kv [gb][rows][2e].
-// grid (gb, heads, query tiles of 64 x splits); 256 threads; head width 16.
-__global__ __launch_bounds__(256) void k_ind_attn16(int rows, int inds, int e, int heads, const float *__restrict__ indq,
-                                                     const float *__restrict__ kv, int kb_per_split,
-                                                     float *__restrict__ part_o, float *__restrict__ part_ml,
-                                                     float *__restrict__ out) {
-    __shared__ float Ks[16][68];
-    __shared__ float Vs[16][68];
-    const int gl = blockIdx.x, h = blockIdx.y;
-    const int ntq = inds / 64, qt = blockIdx.z % ntq, split = blockIdx.z / ntq, splits = gridDim.z / ntq;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g4 = lane >> 4;
-    const int qi = qt * 64 + wave * 16 + r16;
-    const float4 qv = *reinterpret_cast<const float4 *>(indq + (size_t)qi * e + h * 16 + 4 * g4);
-    const float qa[4] = {qv.x, qv.y, qv.z, qv.w};
-    const int n_kb = (rows + 63) / 64;
-    const int kb0 = split * kb_per_split, kb1 = min(n_kb, kb0 + kb_per_split);
-    const float *base = kv + (size_t)gl * rows * 2 * e;
-    float m = -INFINITY, l = 0.0f;
-    floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const int lk = tid >> 2, c4 = (tid & 3) * 4;
-    for (int kb = kb0; kb < kb1; kb++) {
-        const int key0 = kb * 64;
-        float4 kk = make_float4(0.0f, 0.0f, 0.0f, 0.0f), vv = kk;
-        if (key0 + lk < rows) {
-            const float *row = base + (size_t)(key0 + lk) * 2 * e + h * 16 + c4;
-            kk = *reinterpret_cast<const float4 *>(row);
-            vv = *reinterpret_cast<const float4 *>(row + e);
+// The inducing points' queries indq [inds][e] over one group's cells, keys and values from kv [gb][rows][2e]; head width
+// 16. A workgroup takes one group's head over a range of cells, wavefront w its inducing points 32 w .. of the 128 from
+// 128 (blockIdx.z) on: blocks of 128 cells are staged in LDS as split fp16 halves (one block ahead, each thread a key or
+// two coordinates of eight values), then attended as in the fused blocks (attend.hpp), the running maximum carried.
+// Bound by vector work (about ten instructions a score). All heads of a group run on the same XCD, one after another:
+// a row's 2 e floats are read 64 bytes a head, and the heads share the lines in that XCD's L2.
+constexpr int IND_NT = 128, IND_BUF = IND_NT * 128 + 2 * IND_NT * 32;  // a staged block and its rows of ones
+__global__ __launch_bounds__(256, 3) void k_ind_attn16(int gb, int rows, int inds, int e, int heads,
+                                                        const float *__restrict__ indq, const float *__restrict__ kv,
+                                                        int per_split, float *__restrict__ part_o,
+                                                        float *__restrict__ part_ml, float *__restrict__ out) {
+    constexpr int NT = IND_NT, STAGED = NT * 128;
+    __shared__ __align__(1024) uint8_t lds[2 * IND_BUF];
+    __shared__ float red[2][2][2];  // [block parity][keys, values][wavefront of the half]
+    __shared__ int shs[2][2];       // [buffer][keys, values]: the staged block's scales
+    const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3, h = k % heads, gl = k / heads * 8 + xcd;
+    if (gl >= gb) return;
+    const int split = blockIdx.y, splits = gridDim.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r32 = lane & 31, g = lane >> 5;
+    const int qi = blockIdx.z * 128 + wave * 32 + r32, arow = sigma32(r32);
+    const bool live = qi < inds;
+    const int b0 = split * per_split, nb = min((rows + NT - 1) / NT - b0, per_split);
+    const int row0 = b0 * NT;
+
+    // thread t < 128 stages key t, thread 128 + t coordinates 2 (t % 8) and the next of values 8 (t / 8) ..
+    const bool st_key = tid < NT;
+    const int slot = st_key ? tid : (tid - NT) & ~7, sc2 = 2 * (tid & 7), part = st_key ? 0 : 1;
+    // always from the group's own cells (no load behind a branch): past the last cell its again, so that scores need no
+    // mask (those values and ones are zero)
+    const float *src0 = kv + (size_t)gl * rows * 2 * e + 16 * h + (st_key ? 0 : e + sc2);
+    const int per_cell = st_key ? 0 : 1, per_pair = st_key ? 2 : 0;
+    float top = 0.0f;
+    auto stage_load = [&](int b, float (&stv)[16]) {
+        const int at = row0 + b * NT + slot;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float2 v =
+                *reinterpret_cast<const float2 *>(src0 + (size_t)min(at + i * per_cell, rows - 1) * 2 * e + i * per_pair);
+            stv[2 * i] = v.x;
+            stv[2 * i + 1] = v.y;
         }
-        __syncthreads();
-        Ks[c4][lk] = kk.x;
-        Ks[c4 + 1][lk] = kk.y;
-        Ks[c4 + 2][lk] = kk.z;
-        Ks[c4 + 3][lk] = kk.w;
-        Vs[c4][lk] = vv.x;
-        Vs[c4 + 1][lk] = vv.y;
-        Vs[c4 + 2][lk] = vv.z;
-        Vs[c4 + 3][lk] = vv.w;
-        __syncthreads();
-        floatx4 sacc[4];
+    };
+    auto stage_max = [&](int b, const float (&stv)[16]) {
+        float mx = 0.0f;
 #pragma unroll
-        for (int kt = 0; kt < 4; kt++) {
-            sacc[kt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int c = 0; c < 16; c++) mx = fmaxf(mx, fabsf(stv[c]));
+        mx = wave_max(mx);
+        if (lane == 0) red[b & 1][part][wave & 1] = mx;
+    };
+    // the scale is that of the largest value so far, so that it only falls from block to block
+    auto stage_store = [&](int b, const float (&stv)[16]) {
+        const int buf = b & 1;
+        top = fmaxf(top, fmaxf(red[buf][part][0], red[buf][part][1]));
+        const int s = shift_for_max(top);
+        const float f = ldexpf(1.0f, s);
+        if ((tid & (NT - 1)) == 0) shs[buf][part] = s;
+        uint8_t *const at = lds + buf * IND_BUF;
+        const int tg = slot >> 3, left = st_key ? 8 : rows - (row0 + b * NT + slot);  // values of this thread that are there
 #pragma unroll
-            for (int t = 0; t < 4; t++) sacc[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ks[4 * g4 + t][16 * kt + r16], qa[t], sacc[kt], 0, 0, 0);
+        for (int i = 0; i < 2; i++) {
+            float v[8];
+#pragma unroll
+            for (int t = 0; t < 8; t++) v[t] = st_key ? stv[8 * i + t] : t < left ? stv[2 * t + i] : 0.0f;
+            halfx8 hi, lo;
+            split8(v, f, hi, lo);
+            const int cd = sc2 + i;
+            const int place = st_key ? (i * NT + slot) * 16
+                                     : NT * 64 + (tg * 16 + (((cd & 3) | ((cd & 4) << 1) | ((cd & 8) >> 1)) ^ (tg & 15))) * 16;
+            *reinterpret_cast<halfx8 *>(at + place) = hi;
+            *reinterpret_cast<halfx8 *>(at + NT * 32 + place) = lo;
         }
-        float mb = -INFINITY;
+    };
+    float st0[16], stv[16];
+    stage_load(0, st0);
+    if (nb > 1) stage_load(1, stv);
+    pad_rows<NT>(lds + STAGED, tid, NT, min(NT, rows - row0));
+    pad_rows<NT>(lds + IND_BUF + STAGED, tid, NT, min(NT, rows - row0 - NT));
+    // this lane's query, coordinates 8 g .. + 7
+    float qv[8], qmax = 0.0f;
+    load8(indq + (size_t)(live ? qi : 0) * e + h * 16 + 8 * g, qv);
 #pragma unroll
-        for (int kt = 0; kt < 4; kt++)
+    for (int t = 0; t < 8; t++) qmax = fmaxf(qmax, fabsf(qv[t]));
+    const int sq = shift_for_max(fmaxf(qmax, __shfl_xor(qmax, 32, 64)));
+    halfx8 qh, ql;
+    split8(qv, ldexpf(1.0f, sq), qh, ql);
+    stage_max(0, st0);
+    if (nb > 1) stage_max(1, stv);
+    __syncthreads();
+    stage_store(0, st0);
+
+    const bool one = (r32 & 27) == 16;
+    const int kb = (g * NT + arow) * 16;
+    const int vb = one ? STAGED + 16 * g : NT * 64 + 256 * g + 16 * ((r32 & 15) ^ g);
+    float ref = -INFINITY;
+    floatx16 o;
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                if (key0 + 16 * kt + 4 * g4 + v >= rows) sacc[kt][v] = -INFINITY;
-                mb = fmaxf(mb, sacc[kt][v]);
-            }
-        mb = fmaxf(mb, __shfl_xor(mb, 16, 64));
-        mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
-        const float mnew = fmaxf(m, mb);
-        const float alpha = fast_exp(m - mnew);
-        float lb = 0.0f;
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                sacc[kt][v] = fast_exp(sacc[kt][v] - mnew);
-                lb += sacc[kt][v];
-            }
-        lb += __shfl_xor(lb, 16, 64);
-        lb += __shfl_xor(lb, 32, 64);
-        l = l * alpha + lb;
-        m = mnew;
-        acc *= alpha;
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++) {
-            const float4 v4 = *reinterpret_cast<const float4 *>(&Vs[r16][16 * kt + 4 * g4]);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.x, sacc[kt][0], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.y, sacc[kt][1], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.z, sacc[kt][2], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.w, sacc[kt][3], acc, 0, 0, 0);
+    for (int v = 0; v < 16; v++) o[v] = 0.0f;
+    int sv = 0;
+    for (int b = 0; b < nb; b++) {
+        const int at = (b & 1) * IND_BUF;
+        __syncthreads();  // block b is staged, block b + 1's maxima are in red; everyone is done with block b - 1
+        const int sk = shs[b & 1][0], sb = shs[b & 1][1];
+        if (b + 1 < nb) {
+            stage_store(b + 1, stv);
+            // the last block's ones, where it is not whole
+            if (rows - row0 - (b + 1) * NT < NT) pad_rows<NT>(lds + (IND_BUF - at) + STAGED, tid, NT, rows - row0 - (b + 1) * NT);
         }
+        if (b + 2 < nb) stage_load(b + 2, stv);
+        __builtin_amdgcn_sched_barrier(0);  // the loads go out here
+        floatx16 sc[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) sc[j] = score_tile<NT>(lds + at + kb, j, qh, ql);
+        if (b > 0) {
+            const float r = ldexpf(1.0f, sb - sv);
+#pragma unroll
+            for (int t = 0; t < 8; t++) o[t] *= r;
+        }
+        sv = sb;
+        attend_tiles<NT, 4, false>(sc, ldexpf(LOG2E, -(sk + sq)), lds, vb + at, ref, o, [](int) {});
+        if (b + 2 < nb) stage_max(b + 2, stv);  // its loads land under the block's attention
     }
+    if (!live) return;
     const size_t qr = (size_t)gl * inds + qi;  // the (group, inducing point) item
+    float *dst;
+    float f;
     if (splits == 1) {
-        const float inv = 1.0f / l;
-        *reinterpret_cast<float4 *>(out + qr * e + h * 16 + 4 * g4) = make_float4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
+        dst = out + qr * e + h * 16 + 8 * g;
+        f = ldexpf(1.0f, -sv) / o[8];
     } else {
-        const size_t nq = (size_t)gridDim.x * inds;
-        const size_t at = ((size_t)split * nq + qr) * heads + h;
-        *reinterpret_cast<float4 *>(part_o + at * 16 + 4 * g4) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-        if (g4 == 0) {
-            part_ml[at * 2] = m;
-            part_ml[at * 2 + 1] = l;
+        const size_t at = ((size_t)split * gb * inds + qr) * heads + h;
+        dst = part_o + at * 16 + 8 * g;
+        f = ldexpf(1.0f, -sv);
+        if (g == 0) {
+            part_ml[at * 2] = ref;
+            part_ml[at * 2 + 1] = o[8];
         }
     }
+    *reinterpret_cast<float4 *>(dst) = make_float4(o[0] * f, o[1] * f, o[2] * f, o[3] * f);
+    *reinterpret_cast<float4 *>(dst + 4) = make_float4(o[4] * f, o[5] * f, o[6] * f, o[7] * f);
+}
+
+// The splits of k_ind_attn16 merged: thread t four coordinates of item t / 4 ((group, inducing point, head), 16 floats of
+// out in that order; at least one split, every one with keys).
+__global__ __launch_bounds__(256) void k_ind_merge(int items, int splits, const float *__restrict__ part_o,
+                                                    const float *__restrict__ part_ml, float *__restrict__ out) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x, item = i >> 2;
+    if (item >= (size_t)items) return;
+    float top = -INFINITY;
+    for (int s = 0; s < splits; s++) top = fmaxf(top, part_ml[((size_t)s * items + item) * 2]);
+    float l = 0.0f;
+    float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int s = 0; s < splits; s++) {
+        const size_t at = (size_t)s * items + item;
+        const float f = exp2_hw(part_ml[at * 2] - top);
+        const float4 v = reinterpret_cast<const float4 *>(part_o)[at * 4 + (i & 3)];
+        l += part_ml[at * 2 + 1] * f;
+        o.x += v.x * f;
+        o.y += v.y * f;
+        o.z += v.z * f;
+        o.w += v.w * f;
+    }
+    reinterpret_cast<float4 *>(out)[i] = make_float4(o.x / l, o.y / l, o.z / l, o.w / l);
 }
 
 // Any head width (the tiny test models): one thread per (group, inducing point, head), streaming over the rows.
@@ -243,9 +313,6 @@ __global__ __launch_bounds__(256) void k_regroup(int rows, int g, int e, const f
     reinterpret_cast<float4 *>(dst)[cell * e4 + o] = reinterpret_cast<const float4 *>(src)[from * e4 + o];
 }
 
-void merge_splits(hipStream_t s, int nq, int d, int heads, int splits, const float *part_o, const float *part_ml,
-                  float *out);
-
 // ---- launchers ---------------------------------------------------------------------------------------------
 void fit_cells(hipStream_t s, const tah_weights *w, const float *x, int rows, int features, int g0, int gb, float *cells) {
     if (w->group > 8 || w->group < 1) throw ArgError{"column stage: feature group size must be 1..8"};
@@ -260,6 +327,13 @@ void add_y_cells(hipStream_t s, const tah_weights *w, const float *y, int rows, 
     const size_t count = (size_t)gb * rows * w->e;
     hipLaunchKernelGGL(k_add_y, blocks_of(count), dim3(256), 0, s, rows, gb, w->e, w->max_classes, digits, divisor, base, y,
                        w->col_y, cells);
+    TAH_LAUNCHED();
+}
+
+// rows [rows][d] += the in-context stage's target embedding (Model::add_y, src/model.rs:188-200).
+void add_y_rows(hipStream_t s, const tah_weights *w, const float *y, int rows, float *h) {
+    hipLaunchKernelGGL(k_add_y, blocks_of((size_t)rows * w->d), dim3(256), 0, s, rows, 1, w->d, w->max_classes, 1, 1, 1, y,
+                       w->icl_y, h);
     TAH_LAUNCHED();
 }
 
@@ -299,13 +373,14 @@ void tokens_gmajor(hipStream_t s, const tah_weights *w, int rb, int r0, int rows
     TAH_LAUNCHED();
 }
 
+// Ranges of cells a group's head is split into, in blocks of 128: about 4,096 workgroups in all (768 run at once), at
+// least two blocks each.
 static int ind_splits(const tah_weights *w, int rows, int gb) {
-    const int n_kb = (rows + 63) / 64;
-    const int tiles = gb * w->col_heads * std::max(1, w->inds / 64);
-    int want = std::max(1, 1024 / std::max(1, tiles));
-    want = std::min(want, std::max(1, n_kb / 2));
-    const int per = (n_kb + want - 1) / want;
-    return (n_kb + per - 1) / per;
+    const int blocks = (rows + IND_NT - 1) / IND_NT;
+    const int tiles = gb * w->col_heads * ((w->inds + 127) / 128);
+    const int want = std::min(std::max(1, 4096 / std::max(1, tiles)), std::max(1, blocks / 2));
+    const int per = (blocks + want - 1) / want;
+    return (blocks + per - 1) / per;
 }
 
 static bool ind_mfma(const tah_weights *w) { return w->e / w->col_heads == 16 && w->inds % 64 == 0; }
@@ -329,14 +404,17 @@ void ind_attention(hipStream_t s, const tah_weights *w, int rows, int gb, const 
         return;
     }
     const int splits = ind_splits(w, rows, gb);
-    const int n_kb = (rows + 63) / 64;
-    const int per = (n_kb + splits - 1) / splits;
+    const int per = ((rows + IND_NT - 1) / IND_NT + splits - 1) / splits;
     float *part_o = splits > 1 ? static_cast<float *>(work) : nullptr;
     float *part_ml = splits > 1 ? part_o + (size_t)splits * gb * inds * heads * (e / heads) : nullptr;
-    hipLaunchKernelGGL(k_ind_attn16, dim3(gb, heads, (inds / 64) * splits), dim3(256), 0, s, rows, inds, e, heads, indq, kv,
-                       per, part_o, part_ml, out);
+    const dim3 grid((gb + 7) / 8 * 8 * heads, splits, (inds + 127) / 128);
+    hipLaunchKernelGGL(k_ind_attn16, grid, dim3(256), 0, s, gb, rows, inds, e, heads, indq, kv, per, part_o, part_ml, out);
     TAH_LAUNCHED();
-    if (splits > 1) merge_splits(s, gb * inds, e, heads, splits, part_o, part_ml, out);
+    if (splits > 1) {
+        const int items = gb * inds * heads;
+        hipLaunchKernelGGL(k_ind_merge, blocks_of((size_t)items * 4), dim3(256), 0, s, items, splits, part_o, part_ml, out);
+        TAH_LAUNCHED();
+    }
 }
 
 }  // namespace tah
