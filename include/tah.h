@@ -257,6 +257,13 @@ typedef int (*tah_layer_sink)(void *ctx, int32_t layer, const uint8_t *records, 
  * exact f32 keys and values, and the output projection and feed-forward update h. */
 int tah_in_context(tah_dev *dev, const tah_weights *w, const float *h, int32_t rows, const float *scales,
                    int32_t kv_format, int32_t chunk, tah_layer_sink sink, void *ctx);
+/* tah_fit_represent and tah_in_context of a member with one in-context problem over its whole table and one label digit
+ * of base `base` (fit_raw, src/fit.rs:285-752) in one call, the representations kept on the card between them and the
+ * target's embedding added there (src/fit.rs:577-585): col_kv_out and the sink receive what the two calls give. icl_scales
+ * [icl_layers][d] as tah_in_context's scales. A class outside [0, max_classes) fails with TAH_E_ARG. */
+int tah_fit(tah_dev *dev, const tah_weights *w, const float *x, const float *y, int32_t rows, int32_t features,
+            int32_t base, const float *ind_scales, const float *icl_scales, int32_t kv_format, int32_t chunk,
+            float *col_kv_out, tah_layer_sink sink, void *ctx);
 
 /* ---- the regression head: QuantileDist (src/table.rs:292-346) ---------------------------------------------------
  *

@@ -116,6 +116,8 @@ SIGNATURES = {
                                   ctypes.c_int32, F32P]),
     "tah_in_context": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, F32P, ctypes.c_int32, F32P, ctypes.c_int32,
                                       ctypes.c_int32, LAYER_SINK, ctypes.c_void_p]),
+    "tah_fit": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, F32P, F32P, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
+                               F32P, F32P, ctypes.c_int32, ctypes.c_int32, F32P, LAYER_SINK, ctypes.c_void_p]),
     "tah_column_batch": (ctypes.c_size_t, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32]),
     "tah_columns": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, F32P, ctypes.c_int32, ctypes.c_int32, F32P, F32P]),
     "tah_row_batch": (ctypes.c_size_t, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32]),

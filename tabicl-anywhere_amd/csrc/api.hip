@@ -7,6 +7,8 @@
 #include <initializer_list>
 #include <memory>
 #include <new>
+#include <system_error>
+#include <thread>
 
 #include "common.hpp"
 
@@ -908,13 +910,11 @@ extern "C" int tah_quantile_stats(tah_dev *dev, const float *q, int32_t rows, in
     });
 }
 
-// The device's two pinned staging buffers for records on their way to a sink, at least `bytes` each.
+// The device's two pinned staging buffers for records and column caches on their way to the host, at least `bytes` each.
 static void staging(tah_dev *dev, size_t bytes) {
     for (int i = 0; i < 2; i++)
         if (!dev->copied[i]) TAH_HIP(hipEventCreateWithFlags(&dev->copied[i], hipEventDisableTiming));
     if (dev->pinned_bytes >= bytes) return;
-    // a call that failed part-way may have left copies into them queued
-    TAH_HIP(hipStreamSynchronize(dev->stream));
     for (int i = 0; i < 2; i++) {
         if (dev->pinned[i]) TAH_HIP(hipHostFree(dev->pinned[i]));
         dev->pinned[i] = nullptr;
@@ -924,75 +924,154 @@ static void staging(tah_dev *dev, size_t bytes) {
     dev->pinned_bytes = bytes;
 }
 
+// The side stream in use by one call: what is queued on it is finished before the call's buffers (loans taken before
+// this) go back or a staging buffer is used again, also where the call fails part-way.
+struct SideWork {
+    tah_dev *dev;
+    explicit SideWork(tah_dev *d) : dev(d) {}
+    ~SideWork() { (void)hipStreamSynchronize(dev->side); }
+    // what is queued on the main stream up to here runs before what the side stream is given next
+    void follow_main() {
+        TAH_HIP(hipEventRecord(dev->fork_ev, dev->stream));
+        TAH_HIP(hipStreamWaitEvent(dev->side, dev->fork_ev, 0));
+    }
+};
+
+// bytes from one host buffer to another, sliced over a few threads when large (one thread copies to pages it touches
+// for the first time at about 10 GB/s, less than the card delivers them).
+static void host_copy(uint8_t *dst, const uint8_t *src, size_t bytes) {
+    constexpr size_t SLICE = 2 << 20;
+    const size_t n = std::min<size_t>(8, bytes / SLICE);
+    if (n < 2) {
+        std::memcpy(dst, src, bytes);
+        return;
+    }
+    const size_t step = (bytes / n + 4095) & ~size_t(4095);
+    std::vector<std::thread> threads;
+    threads.reserve(n);
+    size_t at = step;  // the first slice is this thread's
+    try {
+        for (; at < bytes; at += step) {
+            const size_t k = std::min(step, bytes - at);
+            threads.emplace_back([=] { std::memcpy(dst + at, src + at, k); });
+        }
+    } catch (const std::system_error &) {  // no more threads: the rest here
+        std::memcpy(dst + at, src + at, bytes - at);
+    }
+    std::memcpy(dst, src, std::min(step, bytes));
+    for (auto &t : threads) t.join();
+}
+
+// Device memory to the caller's (pageable) memory through the pinned staging buffers, on the side stream: each piece's
+// copy to the host runs while the piece before it is copied on. 59 MB straight to pageable memory took 6 ms.
+static void copy_out(tah_dev *dev, void *dst, const void *src, size_t bytes) {
+    staging(dev, std::min<size_t>(bytes, 16 << 20));
+    const size_t piece = std::min<size_t>(dev->pinned_bytes, 16 << 20);
+    const size_t n = (bytes + piece - 1) / piece;
+    for (size_t i = 0; i <= n; i++) {
+        if (i < n) {
+            TAH_HIP(hipMemcpyAsync(dev->pinned[i & 1], static_cast<const uint8_t *>(src) + i * piece,
+                                   std::min(piece, bytes - i * piece), hipMemcpyDeviceToHost, dev->side));
+            TAH_HIP(hipEventRecord(dev->copied[i & 1], dev->side));
+        }
+        if (i > 0) {
+            TAH_HIP(hipEventSynchronize(dev->copied[(i - 1) & 1]));
+            host_copy(static_cast<uint8_t *>(dst) + (i - 1) * piece,
+                      static_cast<const uint8_t *>(dev->pinned[(i - 1) & 1]), std::min(piece, bytes - (i - 1) * piece));
+        }
+    }
+}
+
+static void check_in_context(int rows, int kv_format, int chunk) {
+    if (rows <= 0 || chunk <= 0 || kv_format < 0 || kv_format > 2) throw ArgError{"in_context: bad rows, chunk or format"};
+}
+
+// The in-context stage of a fit from the rows h (on the card, taken over as working memory).
+static void in_context_fit_on(tah_dev *dev, const tah_weights *w, float *h, int rows, const float *scales, int kv_format,
+                              int chunk, tah_layer_sink sink, void *ctx) {
+    const int d = w->d, L = w->icl_layers;
+    const int ff = icl_mid(w);
+    const size_t n = (size_t)rows * d;
+    const size_t lbytes = layer_bytes(kv_format, rows, chunk, d);
+    hipStream_t s = dev->stream;
+    Loans loans(dev);
+    float *t = loans.take<float>(n), *q = loans.take<float>(n);
+    float *att = loans.take<float>(n), *kv = loans.take<float>(2 * n), *rec32 = loans.take<float>(2 * n);
+    float *mid = loans.take<float>((size_t)rows * ff), *sc = loans.take<float>((size_t)L * d);
+    uint8_t *stored[2];  // layer l's records are copied out of stored[l % 2]
+    stored[0] = kv_format == TAH_KV_F32 ? reinterpret_cast<uint8_t *>(rec32) : loans.take<uint8_t>(lbytes);
+    const AttnShape a{rows, rows, chunk, d, w->icl_heads, TAH_KV_F32};
+    void *work = loans.take<uint8_t>(attention_work_bytes(a));
+    KvImages img;
+    const bool use_img = rows >= TAH_SPLIT16_MIN_Q && kv_images_apply(TAH_KV_F32, d, w->icl_heads);
+    if (use_img)
+        img = kv_images_at(loans.take<uint8_t>(kv_images_bytes(rows, chunk, w->icl_heads, TAH_KV_F32)), rows, chunk,
+                           w->icl_heads, TAH_KV_F32);
+    // A second buffer where the budget leaves room for it, so that a layer's records leave the card while it works on
+    // the next layer (10,000 rows in f32: 41 MB, 0.74 ms a layer beside 0.85 ms of kernels; with one buffer the next
+    // layer's records wait for the copy).
+    const size_t used = busy_bytes(dev->pool), room = dev->pool.budget > used ? dev->pool.budget - used : 0;
+    const bool two = loan_raw(lbytes) <= room;
+    stored[1] = two ? loans.take<uint8_t>(lbytes) : stored[0];
+    staging(dev, lbytes);
+    SideWork side(dev);
+    TAH_HIP(hipMemcpyAsync(sc, scales, sizeof(float) * L * d, hipMemcpyHostToDevice, s));
+    for (int l = 0; l < L; l++) {
+        const DevBlock &b = w->icl[l];
+        uint8_t *out = stored[l & 1];
+        float *r32 = kv_format == TAH_KV_F32 ? reinterpret_cast<float *>(out) : rec32;
+        // keys and values of every row, stored (src/fit.rs:627-663); the layer norms inside the products' kernels
+        // where they take them (the split-K kernels from 1,025 rows), else into t first
+        dense(s, rows, 2 * d, d, h, d, b.in_w + (size_t)d * d, b.in_s.rows(d), b.in_b + d, kv, 2 * d, EPI_NONE,
+              nullptr, 0, b.n1w, b.n1b, t);
+        // the copy of the records last in this buffer (layer l - 2's, with one buffer l - 1's) comes before these
+        if (l >= (two ? 2 : 1)) TAH_HIP(hipStreamWaitEvent(s, dev->copied[(l - (two ? 2 : 1)) & 1], 0));
+        to_records(s, rows, d, chunk, kv, r32);
+        if (kv_format != TAH_KV_F32) pack(s, rows, d, chunk, kv_format, r32, out);
+        // layer l's records into staging buffer l % 2 (the sink read layer l - 2's there before this was queued)
+        side.follow_main();
+        TAH_HIP(hipMemcpyAsync(dev->pinned[l & 1], out, lbytes, hipMemcpyDeviceToHost, dev->side));
+        TAH_HIP(hipEventRecord(dev->copied[l & 1], dev->side));
+        const bool last = l + 1 == L;
+        if (!last) {
+            // every row attends to all rows over the exact keys and values, then the rest of the block
+            // (src/fit.rs:667-744)
+            dense(s, rows, d, d, h, d, b.in_w, b.in_s.rows(0), b.in_b, q, d, EPI_NONE, nullptr, 0, b.n1w, b.n1b, t);
+            query_modulate(s, rows, b, sc + (size_t)l * d, q, mid);
+            if (use_img)
+                kv_images(s, rows, chunk, d, w->icl_heads, TAH_KV_F32, reinterpret_cast<const uint8_t *>(r32), img);
+            attention(s, a, q, reinterpret_cast<const uint8_t *>(r32), att, work, use_img ? &img : nullptr);
+            dense(s, rows, d, d, att, d, b.out_w, b.out_s, b.out_b, h, d, EPI_RESID, h, d);
+            dense(s, rows, b.ff, d, h, d, b.l1w, b.l1_s, b.l1b, mid, b.ff, EPI_GELU, nullptr, 0, b.n2w, b.n2b, t);
+            dense(s, rows, d, b.ff, mid, b.ff, b.l2w, b.l2_s, b.l2b, h, d, EPI_RESID, h, d);
+        }
+        // the card works on layer l (queued above) while the sink takes layer l - 1's records
+        if (l > 0) {
+            TAH_HIP(hipEventSynchronize(dev->copied[(l - 1) & 1]));
+            const int rc = sink(ctx, l - 1, static_cast<const uint8_t *>(dev->pinned[(l - 1) & 1]), lbytes);
+            if (rc != 0) {
+                TAH_HIP(hipStreamSynchronize(s));
+                throw SinkError{rc};
+            }
+        }
+    }
+    TAH_HIP(hipEventSynchronize(dev->copied[(L - 1) & 1]));
+    const int rc = sink(ctx, L - 1, static_cast<const uint8_t *>(dev->pinned[(L - 1) & 1]), lbytes);
+    TAH_HIP(hipStreamSynchronize(s));
+    if (rc != 0) throw SinkError{rc};
+    dev->stages++;
+}
+
 extern "C" int tah_in_context(tah_dev *dev, const tah_weights *w, const float *h_host, int32_t rows, const float *scales,
                               int32_t kv_format, int32_t chunk, tah_layer_sink sink, void *ctx) {
     if (!w || !h_host || !scales || !sink) return TAH_E_ARG;
     return guarded(dev, [&] {
-        if (rows <= 0 || chunk <= 0 || kv_format < 0 || kv_format > 2) throw ArgError{"in_context: bad rows, chunk or format"};
-        const int d = w->d, L = w->icl_layers;
-        const int ff = icl_mid(w);
-        const size_t n = (size_t)rows * d;
-        const size_t lbytes = layer_bytes(kv_format, rows, chunk, d);
-        hipStream_t s = dev->stream;
+        check_in_context(rows, kv_format, chunk);
         Loans loans(dev);
-        float *h = loans.take<float>(n), *t = loans.take<float>(n), *q = loans.take<float>(n);
-        float *att = loans.take<float>(n), *kv = loans.take<float>(2 * n), *rec32 = loans.take<float>(2 * n);
-        float *mid = loans.take<float>((size_t)rows * ff), *sc = loans.take<float>((size_t)L * d);
-        uint8_t *recq = kv_format == TAH_KV_F32 ? nullptr : loans.take<uint8_t>(lbytes);
-        const AttnShape a{rows, rows, chunk, d, w->icl_heads, TAH_KV_F32};
-        void *work = loans.take<uint8_t>(attention_work_bytes(a));
-        KvImages img;
-        const bool use_img = rows >= TAH_SPLIT16_MIN_Q && kv_images_apply(TAH_KV_F32, d, w->icl_heads);
-        if (use_img)
-            img = kv_images_at(loans.take<uint8_t>(kv_images_bytes(rows, chunk, w->icl_heads, TAH_KV_F32)), rows, chunk,
-                               w->icl_heads, TAH_KV_F32);
-        staging(dev, lbytes);
-        TAH_HIP(hipMemcpyAsync(h, h_host, n * sizeof(float), hipMemcpyHostToDevice, s));
-        TAH_HIP(hipMemcpyAsync(sc, scales, sizeof(float) * L * d, hipMemcpyHostToDevice, s));
-        for (int l = 0; l < L; l++) {
-            const DevBlock &b = w->icl[l];
-            // keys and values of every row, stored (src/fit.rs:627-663); the layer norms inside the products' kernels
-            // where they take them (the split-K kernels from 1,025 rows), else into t first
-            dense(s, rows, 2 * d, d, h, d, b.in_w + (size_t)d * d, b.in_s.rows(d), b.in_b + d, kv, 2 * d, EPI_NONE,
-                  nullptr, 0, b.n1w, b.n1b, t);
-            to_records(s, rows, d, chunk, kv, rec32);
-            const uint8_t *stored = reinterpret_cast<const uint8_t *>(rec32);
-            if (kv_format != TAH_KV_F32) {
-                pack(s, rows, d, chunk, kv_format, rec32, recq);
-                stored = recq;
-            }
-            // layer l's records into staging buffer l % 2 (the sink read layer l - 2's there before this was queued)
-            TAH_HIP(hipMemcpyAsync(dev->pinned[l & 1], stored, lbytes, hipMemcpyDeviceToHost, s));
-            TAH_HIP(hipEventRecord(dev->copied[l & 1], s));
-            const bool last = l + 1 == L;
-            if (!last) {
-                // every row attends to all rows over the exact keys and values, then the rest of the block
-                // (src/fit.rs:667-744)
-                dense(s, rows, d, d, h, d, b.in_w, b.in_s.rows(0), b.in_b, q, d, EPI_NONE, nullptr, 0, b.n1w, b.n1b, t);
-                query_modulate(s, rows, b, sc + (size_t)l * d, q, mid);
-                if (use_img)
-                    kv_images(s, rows, chunk, d, w->icl_heads, TAH_KV_F32, reinterpret_cast<const uint8_t *>(rec32), img);
-                attention(s, a, q, reinterpret_cast<const uint8_t *>(rec32), att, work, use_img ? &img : nullptr);
-                dense(s, rows, d, d, att, d, b.out_w, b.out_s, b.out_b, h, d, EPI_RESID, h, d);
-                dense(s, rows, b.ff, d, h, d, b.l1w, b.l1_s, b.l1b, mid, b.ff, EPI_GELU, nullptr, 0, b.n2w, b.n2b, t);
-                dense(s, rows, d, b.ff, mid, b.ff, b.l2w, b.l2_s, b.l2b, h, d, EPI_RESID, h, d);
-            }
-            // the card works on layer l (queued above) while the sink takes layer l - 1's records; on the stream the
-            // copy of layer l's records runs before layer l + 1's keys overwrite rec32
-            if (l > 0) {
-                TAH_HIP(hipEventSynchronize(dev->copied[(l - 1) & 1]));
-                const int rc = sink(ctx, l - 1, static_cast<const uint8_t *>(dev->pinned[(l - 1) & 1]), lbytes);
-                if (rc != 0) {
-                    TAH_HIP(hipStreamSynchronize(s));  // nothing queued is left touching the staging buffers
-                    throw SinkError{rc};
-                }
-            }
-        }
-        TAH_HIP(hipEventSynchronize(dev->copied[(L - 1) & 1]));
-        const int rc = sink(ctx, L - 1, static_cast<const uint8_t *>(dev->pinned[(L - 1) & 1]), lbytes);
-        TAH_HIP(hipStreamSynchronize(s));
-        if (rc != 0) throw SinkError{rc};
-        dev->stages++;
+        const size_t n = (size_t)rows * w->d;
+        float *h = loans.take<float>(n);
+        TAH_HIP(hipMemcpyAsync(h, h_host, n * sizeof(float), hipMemcpyHostToDevice, dev->stream));
+        in_context_fit_on(dev, w, h, rows, scales, kv_format, chunk, sink, ctx);
         return TAH_OK;
     });
 }
@@ -1326,86 +1405,125 @@ static void check_fit_weights(const tah_weights *w) {
         throw ArgError{"fit: the weights lack the column or row stage (upload them with the fitting blocks)"};
 }
 
+// The column and row stages of a fit: the rows' representations into reps (on the card; with labels the in-context
+// stage's target embedding added), the column cache to col_kv_out. The cache leaves the card while it works on the row
+// stage.
+static void fit_represent_on(tah_dev *dev, const tah_weights *w, const float *x, const float *y, int rows, int features,
+                             const int32_t *bases, int digits, const float *ind_scales, float *col_kv_out, float *reps,
+                             bool labels) {
+    const int e = w->e, inds = w->inds, nb = w->col_blocks, d = w->d;
+    const int T = w->cls + features;
+    const size_t per = 2 * (size_t)e * inds, gstride = (size_t)digits * nb * per;
+    hipStream_t s = dev->stream;
+    Loans keep(dev);
+    float *xd = keep.take<float>((size_t)rows * features), *yd = keep.take<float>(rows);
+    float *sc = keep.take<float>((size_t)nb * e), *indq = keep.take<float>((size_t)nb * inds * e);
+    float *it = keep.take<float>((size_t)inds * e);
+    float *col_kv = keep.take<float>((size_t)features * gstride);
+    float *emb = keep.take<float>((size_t)features * rows * e);
+    SideWork side(dev);
+    TAH_HIP(hipMemcpyAsync(xd, x, sizeof(float) * rows * features, hipMemcpyHostToDevice, s));
+    TAH_HIP(hipMemcpyAsync(yd, y, sizeof(float) * rows, hipMemcpyHostToDevice, s));
+    TAH_HIP(hipMemcpyAsync(sc, ind_scales, sizeof(float) * nb * e, hipMemcpyHostToDevice, s));
+    // the inducing points' queries, once per block, scaled for all rows (src/fit.rs:300-313)
+    size_t qfloats = 0;
+    for (auto &b : w->col_a1) qfloats = std::max(qfloats, query_scratch_floats(inds, b));
+    Loans qloan(dev);
+    float *qscr = qloan.take<float>(std::max<size_t>(qfloats, 1));
+    for (int bi = 0; bi < nb; bi++) {
+        const DevBlock &a1 = w->col_a1[bi];
+        float *qb = indq + (size_t)bi * inds * e;
+        layer_norm(s, inds, e, w->col_ind + (size_t)bi * inds * e, e, a1.n1w, a1.n1b, it, e);
+        gemm(s, inds, e, e, it, e, a1.in_w, a1.in_b, qb, e, EPI_NONE, nullptr, 0);
+        query_modulate(s, inds, a1, sc + (size_t)bi * e, qb, qscr);
+    }
+    // feature groups in batches that fit the working memory
+    const int gb = batch_rows(dev, features, [&](int g) {
+        const size_t M = (size_t)g * rows;
+        return column_bufs_bytes(w, rows, g) + (digits > 1 ? loan_bytes({M * e, M * e}) : 0);
+    });
+    for (int g0 = 0; g0 < features; g0 += gb) {
+        const int g = std::min(gb, features - g0);
+        const size_t M = (size_t)g * rows;
+        Loans loans(dev);
+        float *cells = emb + (size_t)g0 * rows * e;
+        const ColumnBufs cb = column_bufs(w, rows, g, loans);
+        float *plain = digits > 1 ? loans.take<float>(M * e) : nullptr;
+        float *sum = digits > 1 ? loans.take<float>(M * e) : nullptr;
+        fit_cells(s, w, xd, rows, features, g0, g, cells);
+        if (digits > 1) {
+            TAH_HIP(hipMemcpyAsync(plain, cells, M * e * sizeof(float), hipMemcpyDeviceToDevice, s));
+            TAH_HIP(hipMemsetAsync(sum, 0, M * e * sizeof(float), s));
+        }
+        for (int dg = 0; dg < digits; dg++) {
+            if (dg > 0) TAH_HIP(hipMemcpyAsync(cells, plain, M * e * sizeof(float), hipMemcpyDeviceToDevice, s));
+            int divisor = 1;
+            for (int k = dg + 1; k < digits; k++) divisor *= bases[k];
+            add_y_cells(s, w, yd, rows, g, digits, divisor, bases[dg], cells);
+            column_blocks(s, w, cells, rows, g, indq, col_kv, gstride, (size_t)dg * nb * per, g0, cb);
+            if (digits > 1) add_to(s, M * e, cells, sum);
+        }
+        if (digits > 1) scale_by(s, M * e, sum, 1.0f / (float)digits, cells);
+    }
+    side.follow_main();  // the column cache is whole
+    // the row stage in batches of rows (src/fit.rs:516-539)
+    const RopeTabs tabs = rope_tables(w, T);
+    const int rb = batch_rows(dev, rows, [&](int k) {
+        return loan_bytes({(size_t)k * T * e, row_stage_floats(w, k, T)});
+    });
+    for (int r0 = 0; r0 < rows; r0 += rb) {
+        const int k = std::min(rb, rows - r0);
+        Loans loans(dev);
+        float *tok = loans.take<float>((size_t)k * T * e);
+        float *scratch = loans.take<float>(row_stage_floats(w, k, T));
+        tokens_gmajor(s, w, k, r0, rows, features, emb, tok);
+        row_stage(s, w, tok, k, T, tabs.cos, tabs.sin, reps + (size_t)r0 * d, scratch);
+    }
+    if (labels) add_y_rows(s, w, yd, rows, reps);
+    copy_out(dev, col_kv_out, col_kv, sizeof(float) * features * gstride);
+}
+
+static void check_fit_sizes(int rows, int features, const int32_t *bases, int digits) {
+    if (rows <= 0 || features <= 0 || digits <= 0) throw ArgError{"fit: bad rows, features or digits"};
+    for (int i = 0; i < digits; i++)
+        if (bases[i] <= 0) throw ArgError{"fit: label digit bases must be positive"};
+}
+
 extern "C" int tah_fit_represent(tah_dev *dev, const tah_weights *w, const float *x, const float *y, int32_t rows,
                                  int32_t features, const int32_t *bases, int32_t digits, const float *ind_scales,
                                  float *col_kv_out, float *reps_out) {
     if (!w || !x || !y || !bases || !ind_scales || !col_kv_out || !reps_out) return TAH_E_ARG;
     return guarded(dev, [&] {
-        if (rows <= 0 || features <= 0 || digits <= 0) throw ArgError{"fit: bad rows, features or digits"};
+        check_fit_sizes(rows, features, bases, digits);
         check_fit_weights(w);
-        for (int i = 0; i < digits; i++)
-            if (bases[i] <= 0) throw ArgError{"fit: label digit bases must be positive"};
-        const int e = w->e, inds = w->inds, nb = w->col_blocks, d = w->d;
-        const int T = w->cls + features;
-        const size_t per = 2 * (size_t)e * inds, gstride = (size_t)digits * nb * per;
-        hipStream_t s = dev->stream;
         Loans keep(dev);
-        float *xd = keep.take<float>((size_t)rows * features), *yd = keep.take<float>(rows);
-        float *sc = keep.take<float>((size_t)nb * e), *indq = keep.take<float>((size_t)nb * inds * e);
-        float *it = keep.take<float>((size_t)inds * e);
-        float *col_kv = keep.take<float>((size_t)features * gstride);
-        float *emb = keep.take<float>((size_t)features * rows * e);
-        float *reps = keep.take<float>((size_t)rows * d);
-        TAH_HIP(hipMemcpyAsync(xd, x, sizeof(float) * rows * features, hipMemcpyHostToDevice, s));
-        TAH_HIP(hipMemcpyAsync(yd, y, sizeof(float) * rows, hipMemcpyHostToDevice, s));
-        TAH_HIP(hipMemcpyAsync(sc, ind_scales, sizeof(float) * nb * e, hipMemcpyHostToDevice, s));
-        // the inducing points' queries, once per block, scaled for all rows (src/fit.rs:300-313)
-        size_t qfloats = 0;
-        for (auto &b : w->col_a1) qfloats = std::max(qfloats, query_scratch_floats(inds, b));
-        Loans qloan(dev);
-        float *qscr = qloan.take<float>(std::max<size_t>(qfloats, 1));
-        for (int bi = 0; bi < nb; bi++) {
-            const DevBlock &a1 = w->col_a1[bi];
-            float *qb = indq + (size_t)bi * inds * e;
-            layer_norm(s, inds, e, w->col_ind + (size_t)bi * inds * e, e, a1.n1w, a1.n1b, it, e);
-            gemm(s, inds, e, e, it, e, a1.in_w, a1.in_b, qb, e, EPI_NONE, nullptr, 0);
-            query_modulate(s, inds, a1, sc + (size_t)bi * e, qb, qscr);
-        }
-        // feature groups in batches that fit the working memory
-        const int gb = batch_rows(dev, features, [&](int g) {
-            const size_t M = (size_t)g * rows;
-            return column_bufs_bytes(w, rows, g) + (digits > 1 ? loan_bytes({M * e, M * e}) : 0);
-        });
-        for (int g0 = 0; g0 < features; g0 += gb) {
-            const int g = std::min(gb, features - g0);
-            const size_t M = (size_t)g * rows;
-            Loans loans(dev);
-            float *cells = emb + (size_t)g0 * rows * e;
-            const ColumnBufs cb = column_bufs(w, rows, g, loans);
-            float *plain = digits > 1 ? loans.take<float>(M * e) : nullptr;
-            float *sum = digits > 1 ? loans.take<float>(M * e) : nullptr;
-            fit_cells(s, w, xd, rows, features, g0, g, cells);
-            if (digits > 1) {
-                TAH_HIP(hipMemcpyAsync(plain, cells, M * e * sizeof(float), hipMemcpyDeviceToDevice, s));
-                TAH_HIP(hipMemsetAsync(sum, 0, M * e * sizeof(float), s));
-            }
-            for (int dg = 0; dg < digits; dg++) {
-                if (dg > 0) TAH_HIP(hipMemcpyAsync(cells, plain, M * e * sizeof(float), hipMemcpyDeviceToDevice, s));
-                int divisor = 1;
-                for (int k = dg + 1; k < digits; k++) divisor *= bases[k];
-                add_y_cells(s, w, yd, rows, g, digits, divisor, bases[dg], cells);
-                column_blocks(s, w, cells, rows, g, indq, col_kv, gstride, (size_t)dg * nb * per, g0, cb);
-                if (digits > 1) add_to(s, M * e, cells, sum);
-            }
-            if (digits > 1) scale_by(s, M * e, sum, 1.0f / (float)digits, cells);
-        }
-        // the row stage in batches of rows (src/fit.rs:516-539)
-        const RopeTabs tabs = rope_tables(w, T);
-        const int rb = batch_rows(dev, rows, [&](int k) {
-            return loan_bytes({(size_t)k * T * e, row_stage_floats(w, k, T)});
-        });
-        for (int r0 = 0; r0 < rows; r0 += rb) {
-            const int k = std::min(rb, rows - r0);
-            Loans loans(dev);
-            float *tok = loans.take<float>((size_t)k * T * e);
-            float *scratch = loans.take<float>(row_stage_floats(w, k, T));
-            tokens_gmajor(s, w, k, r0, rows, features, emb, tok);
-            row_stage(s, w, tok, k, T, tabs.cos, tabs.sin, reps + (size_t)r0 * d, scratch);
-        }
-        TAH_HIP(hipMemcpyAsync(col_kv_out, col_kv, sizeof(float) * features * gstride, hipMemcpyDeviceToHost, s));
-        TAH_HIP(hipMemcpyAsync(reps_out, reps, sizeof(float) * rows * d, hipMemcpyDeviceToHost, s));
-        TAH_HIP(hipStreamSynchronize(s));
+        float *reps = keep.take<float>((size_t)rows * w->d);
+        fit_represent_on(dev, w, x, y, rows, features, bases, digits, ind_scales, col_kv_out, reps, false);
+        TAH_HIP(hipMemcpyAsync(reps_out, reps, sizeof(float) * rows * w->d, hipMemcpyDeviceToHost, dev->stream));
+        TAH_HIP(hipStreamSynchronize(dev->stream));
         dev->stages += 2;  // the column and the row stage
+        return TAH_OK;
+    });
+}
+
+extern "C" int tah_fit(tah_dev *dev, const tah_weights *w, const float *x, const float *y, int32_t rows, int32_t features,
+                       int32_t base, const float *ind_scales, const float *icl_scales, int32_t kv_format, int32_t chunk,
+                       float *col_kv_out, tah_layer_sink sink, void *ctx) {
+    if (!w || !x || !y || !ind_scales || !icl_scales || !col_kv_out || !sink) return TAH_E_ARG;
+    return guarded(dev, [&] {
+        check_fit_sizes(rows, features, &base, 1);
+        check_in_context(rows, kv_format, chunk);
+        check_fit_weights(w);
+        if (!w->icl_y) throw ArgError{"fit: the weights lack the in-context target embedding"};
+        // a class's embedding is a row of a table
+        if (w->max_classes > 0)
+            for (int r = 0; r < rows; r++)
+                if (!(y[r] >= 0.0f && y[r] < (float)w->max_classes)) throw ArgError{"fit: a class out of range"};
+        Loans keep(dev);
+        float *reps = keep.take<float>((size_t)rows * w->d);
+        fit_represent_on(dev, w, x, y, rows, features, &base, 1, ind_scales, col_kv_out, reps, true);
+        dev->stages += 2;
+        in_context_fit_on(dev, w, reps, rows, icl_scales, kv_format, chunk, sink, ctx);
         return TAH_OK;
     });
 }

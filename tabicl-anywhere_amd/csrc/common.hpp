@@ -331,6 +331,7 @@ void column_block(hipStream_t s, const tah_weights *w, const DevBlock &b, float 
 
 // The column stage of a fit (fit_stages.hip).
 void fit_cells(hipStream_t s, const tah_weights *w, const float *x, int rows, int features, int g0, int gb, float *cells);
+void add_y_rows(hipStream_t s, const tah_weights *w, const float *y, int rows, float *h);
 void add_y_cells(hipStream_t s, const tah_weights *w, const float *y, int rows, int gb, int digits, int divisor, int base,
                  float *cells);
 void scale_by(hipStream_t s, size_t count, const float *src, float f, float *dst);

@@ -313,6 +313,30 @@ class Gpu:
         if scales.size != m.icl_layers * m.d:
             raise ValueError(f"in_context_fit: scales must be [{m.icl_layers}][{m.d}]")
         rows = h.shape[0]
+        self._with_sink(sink, lambda cb: self._l.tah_in_context(self._h, weights._h, _fp(h), rows, _fp(scales),
+                                                                int(kv_format), int(chunk), cb, None))
+        return True
+
+    def fit(self, weights: "GpuWeights", x, y, base: int, ind_scales, icl_scales, kv_format: int, chunk: int, sink):
+        """`fit_represent` and `in_context_fit` in one call for a member with one in-context problem over its whole
+        table and one label digit (of base `base`), the representations kept on the card in between and the target's
+        embedding added there. `sink` as for `in_context_fit`; returns col_kv [features][1][blocks][2][e][inds]."""
+        m = weights.model
+        x, y = _f32(x), _f32(y).reshape(-1)
+        if x.ndim != 2 or y.size != x.shape[0]:
+            raise ValueError("fit: x must be [rows][features] and y [rows]")
+        rows, features = x.shape
+        ind_scales, icl_scales = _f32(ind_scales), _f32(icl_scales)
+        if ind_scales.size != len(m.col_a1) * m.e or icl_scales.size != m.icl_layers * m.d:
+            raise ValueError(f"fit: ind_scales must be [{len(m.col_a1)}][{m.e}], icl_scales [{m.icl_layers}][{m.d}]")
+        col_kv = np.empty((features, 1, len(m.col_a2), 2, m.e, m.inds), np.float32)
+        self._with_sink(sink, lambda cb: self._l.tah_fit(self._h, weights._h, _fp(x), _fp(y), rows, features, int(base),
+                                                         _fp(ind_scales), _fp(icl_scales), int(kv_format), int(chunk),
+                                                         _fp(col_kv), cb, None))
+        return col_kv
+
+    def _with_sink(self, sink, run) -> None:
+        """run(cb) with sink(layer, records) as the C callback; what the sink raised is raised here."""
         failure = []
 
         def call(_ctx, layer, ptr, nbytes):
@@ -323,12 +347,10 @@ class Gpu:
                 failure.append(exc)
                 return 1
 
-        cb = abi.LAYER_SINK(call)
-        rc = self._l.tah_in_context(self._h, weights._h, _fp(h), rows, _fp(scales), int(kv_format), int(chunk), cb, None)
+        rc = run(abi.LAYER_SINK(call))
         if failure:
             raise failure[0]
         self._check(rc)
-        return True
 
     # device-pointer forms: inputs already in HBM, work left queued on the handle's stream
     def attend_resident_dev(self, vm: "VramModel", layer: int, q_ptr: int, nq: int, out_ptr: int) -> None:

@@ -37,7 +37,7 @@ class Plan:
 
     @classmethod
     def new(cls, max_classes: int, y, classes: int) -> "Plan":
-        y = [float(v) for v in y]
+        y = np.asarray(y, np.float64).tolist()
         mx = max_classes
         if mx == 0 or classes <= mx:
             return cls([max(classes, 1)], [Node(None, list(y), classes, True, list(range(classes)))])

@@ -1,0 +1,137 @@
+"""The inducing points' attention of a fit at the edges of its blocks of 128 cells (one cell, a block less and more one
+cell, splits of uneven length) against the oracle at the stages' tolerance, 5e-5; and the fit in one call (tah_fit)
+against the column, row and in-context calls apart: the same bits, with room for the second record buffer and without,
+and after a sink has stopped one."""
+import numpy as np
+import pytest
+
+import oracle as orc
+from conftest import pkg
+from test_gpu_stages import TOL, say
+
+abi, fit, hip, M = pkg("abi"), pkg("fit"), pkg("hip"), pkg("model")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    g = hip.Gpu(0)
+    yield g
+    g.close()
+
+
+@pytest.fixture(scope="module", params=["clf", "reg"])
+def kind(request):
+    return request.param
+
+
+@pytest.fixture(scope="module")
+def model(kind):
+    return M.Model.random(M.FULL_CLASSIFIER if kind == "clf" else M.FULL_REGRESSOR, seed=2)
+
+
+@pytest.fixture(scope="module")
+def weights(gpu, model):
+    return gpu.weights(model)
+
+
+def table(kind, rows, features):
+    rng = np.random.default_rng([rows, features])
+    y = rng.integers(0, 10, rows) if kind == "clf" else rng.standard_normal(rows)
+    return rng.standard_normal((rows, features)).astype(np.float32), y.astype(np.float32)
+
+
+@pytest.mark.parametrize("rows,features", [(1, 1), (2, 9), (127, 2), (128, 1), (129, 9), (255, 3), (257, 8), (700, 2)])
+def test_inducing_attention(gpu, kind, model, weights, rows, features):
+    say(f"inducing points {kind} rows={rows} features={features}")
+    x, y = table(kind, rows, features)
+    base = 10 if kind == "clf" else model.outputs
+    scales = np.stack([fit.query_scale(b, rows) for b in model.col_a1])
+    col, reps = gpu.fit_represent(weights, x, y, [base], scales)
+    want, emb = orc.fit_columns(model, x, y, [base], 256)
+    err = max(np.abs(col - want).max(), np.abs(reps - orc.fit_rows(model, emb)).max())
+    say("  worst", err)
+    assert err < TOL
+
+
+def apart(gpu, weights, x, y, base, kv_format, chunk):
+    m = weights.model
+    rows = len(x)
+    col, h = gpu.fit_represent(weights, x, y, [base], np.stack([fit.query_scale(b, rows) for b in m.col_a1]))
+    m.add_y(m.t["icl_y"], y, h)
+    layers = []
+    gpu.in_context_fit(weights, h, np.stack([fit.query_scale(b, rows) for b in m.icl]), kv_format, chunk,
+                       lambda l, rec: layers.append(rec.copy()))
+    return col, layers
+
+
+@pytest.mark.parametrize("rows,features,kv_format,chunk", [(70, 3, abi.KV_F32, 256), (300, 12, abi.KV_I8, 100),
+                                                           (1100, 4, abi.KV_F32, 256), (513, 2, abi.KV_I16, 64)])
+def test_fit_in_one_call(gpu, kind, model, weights, rows, features, kv_format, chunk):
+    say(f"fit in one call {kind} rows={rows} format={kv_format}")
+    x, y = table(kind, rows, features)
+    base = 10 if kind == "clf" else model.outputs
+    col, layers = apart(gpu, weights, x, y, base, kv_format, chunk)
+    got = fit.fit_raw(gpu, weights, x, y, base, chunk, kv_format)
+    assert np.array_equal(got.col_kv, col)
+
+    assert len(got.layers[0]) == len(layers) == model.icl_layers
+    if kind == "clf":
+        assert all(np.array_equal(a, b) for a, b in zip(got.layers[0], layers))
+    elif kv_format == abi.KV_F32:
+        # the embedding's multiply and add are one rounding on the card, two on the host: 2^-24 of it, carried on
+        assert max(np.abs(a.view(np.float32) - b.view(np.float32)).max() for a, b in zip(got.layers[0], layers)) < TOL
+
+
+@pytest.mark.parametrize("rows,kv_format", [(300, abi.KV_I8), (1100, abi.KV_F32)])
+def test_records_through_one_buffer(gpu, model, weights, rows, kv_format):
+    """Under the least budget that takes the call there is no room for the second record buffer: the same records."""
+    h = np.random.default_rng(rows).standard_normal((rows, model.d)).astype(np.float32)
+    scales = np.stack([fit.query_scale(b, rows) for b in model.icl])
+
+    def run():
+        layers = []
+        gpu.in_context_fit(weights, h, scales, kv_format, 256, lambda l, rec: layers.append(rec.copy()))
+        return layers
+
+    gpu.release()
+    want = run()
+    budget, low, high, least = gpu.work_budget(), 0, gpu.working()[1], None
+    try:
+        while high - low > 1 << 14:
+            mid = (low + high) // 2
+            gpu.release()
+            gpu.set_work_budget(mid)
+            try:
+                least, high = run(), mid
+            except hip.BudgetError:
+                low = mid
+    finally:
+        gpu.set_work_budget(budget)
+    say(f"  one buffer rows={rows} format={kv_format}: {high} bytes")
+    assert least is not None and all(np.array_equal(a, b) for a, b in zip(least, want))
+
+
+def test_sink_stops_a_fit(gpu, kind, model, weights):
+    x, y = table(kind, 300, 3)
+    base = 10 if kind == "clf" else model.outputs
+    ind = np.stack([fit.query_scale(b, 300) for b in model.col_a1])
+    icl = np.stack([fit.query_scale(b, 300) for b in model.icl])
+    full, seen = [], []
+    gpu.fit(weights, x, y, base, ind, icl, abi.KV_F32, 256, lambda l, rec: full.append(rec.copy()))
+
+    def stop(l, rec):
+        seen.append(rec.copy())
+        if l == 2:
+            raise KeyError("enough")
+
+    with pytest.raises(KeyError):
+        gpu.fit(weights, x, y, base, ind, icl, abi.KV_F32, 256, stop)
+    again = []
+    gpu.fit(weights, x, y, base, ind, icl, abi.KV_F32, 256, lambda l, rec: again.append(rec.copy()))
+    assert len(seen) == 3 and all(np.array_equal(a, b) for a, b in zip(seen, full))
+    assert all(np.array_equal(a, b) for a, b in zip(again, full))
+    if kind == "clf":
+        y[7] = 10.0
+        with pytest.raises(ValueError):
+            gpu.fit(weights, x, y, base, ind, icl, abi.KV_F32, 256, stop)
