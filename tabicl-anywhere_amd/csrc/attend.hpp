@@ -66,8 +66,7 @@ __device__ __forceinline__ void attend_tiles(floatx16 (&sc)[S], float to_log2, c
     for (int j = 0; j < TILES; j++)
 #pragma unroll
         for (int v = 0; v < 16; v++) mx = fmaxf(mx, sc[j][v]);
-    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-    mx = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1])) * to_log2;
+    mx = half_max(mx) * to_log2;
     if (FIRST) {
         ref = mx;
 #pragma unroll

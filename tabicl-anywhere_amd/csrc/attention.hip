@@ -889,7 +889,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_attn_split64(int nq, int rows
         for (int dc = 0; dc < 4; dc++)
 #pragma unroll
             for (int t = 0; t < 8; t++) qmax = fmaxf(qmax, fabsf(qs[dc][t]));
-        qmax = fmaxf(qmax, __shfl_xor(qmax, 32, 64));
+        qmax = half_max(qmax);
         const int eq = shift_for(__float_as_uint(qmax));
 #pragma unroll
         for (int dc = 0; dc < 4; dc++) {

@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256, 1) void k_ff128h(int M, float *__restrict__ x,
                 mx = fmaxf(mx, fabsf(hv));
             }
         }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = half_max(mx);
     const int sh = shift_for_max(mx);
     halfx8 hh8[8], hl8[8];
 #pragma unroll
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(256, 2) void k_rows128(int M, int N, const float *_
         for (int ks = 0; ks < 8; ks++)
 #pragma unroll
             for (int t = 0; t < 8; t++) sum += xv[ks][t];
-        sum += __shfl_xor(sum, 32, 64);
+        sum = half_sum(sum);
         const float mean = sum / 128.0f;
         float sq = 0.0f;
 #pragma unroll
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(256, 2) void k_rows128(int M, int N, const float *_
                 const float dv = xv[ks][t] - mean;
                 sq += dv * dv;
             }
-        sq += __shfl_xor(sq, 32, 64);
+        sq = half_sum(sq);
         const float inv = 1.0f / sqrtf(sq / 128.0f + 1e-5f);
 #pragma unroll
         for (int ks = 0; ks < 8; ks++) {
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(256, 2) void k_rows128(int M, int N, const float *_
     for (int ks = 0; ks < 8; ks++)
 #pragma unroll
         for (int t = 0; t < 8; t++) xmax = fmaxf(xmax, fabsf(xv[ks][t]));
-    xmax = fmaxf(xmax, __shfl_xor(xmax, 32, 64));
+    xmax = half_max(xmax);
     const int sx = shift_for_max(xmax);
     halfx8 xh[8], xl[8];
 #pragma unroll
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(256, 2) void k_cell_block(int n, size_t sr, size_t 
         for (int ks = 0; ks < 8; ks++)
 #pragma unroll
             for (int t = 0; t < 8; t++) sum += xv[ks][t];
-        sum += __shfl_xor(sum, 32, 64);
+        sum = half_sum(sum);
         const float mean = sum / 128.0f;
         float sq = 0.0f;
 #pragma unroll
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(256, 2) void k_cell_block(int n, size_t sr, size_t 
                 const float dv = xv[ks][t] - mean;
                 sq += dv * dv;
             }
-        sq += __shfl_xor(sq, 32, 64);
+        sq = half_sum(sq);
         const float inv = 1.0f / sqrtf(sq / 128.0f + 1e-5f);
 #pragma unroll
         for (int ks = 0; ks < 8; ks++) {
@@ -541,7 +541,7 @@ __global__ __launch_bounds__(256, 2) void k_cell_block(int n, size_t sr, size_t 
     for (int ks = 0; ks < 8; ks++)
 #pragma unroll
         for (int t = 0; t < 8; t++) xmax = fmaxf(xmax, fabsf(xv[ks][t]));
-    xmax = fmaxf(xmax, __shfl_xor(xmax, 32, 64));
+    xmax = half_max(xmax);
     const int sx = shift_for_max(xmax);
     const int arow = sigma32(r32);
 
@@ -590,7 +590,7 @@ __global__ __launch_bounds__(256, 2) void k_cell_block(int n, size_t sr, size_t 
         for (int T = 0; T < 4; T++)
 #pragma unroll
             for (int v = 0; v < 16; v++) qmax = fmaxf(qmax, fabsf(qa[T][v]));
-        sq = shift_for_max(fmaxf(qmax, __shfl_xor(qmax, 32, 64)));
+        sq = shift_for_max(half_max(qmax));
 #pragma unroll
         for (int h = 0; h < 8; h++) {
             float qv[8];

@@ -15,26 +15,43 @@ __device__ __forceinline__ float dpp(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, false));
 }
 
+// op of lanes i and i ^ 16 (rows of sixteen), i and i ^ 32 (halves), in both
+template <class F>
+__device__ __forceinline__ float row_pair(float v, F &&op) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+template <class F>
+__device__ __forceinline__ float half_pair(float v, F &&op) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+
+__device__ __forceinline__ float add2(float a, float b) { return a + b; }
+__device__ __forceinline__ float row_sum(float v) { return row_pair(v, add2); }
+__device__ __forceinline__ float row_max(float v) { return row_pair(v, fmaxf); }
+__device__ __forceinline__ float half_sum(float v) { return half_pair(v, add2); }
+__device__ __forceinline__ float half_max(float v) { return half_pair(v, fmaxf); }
+
+// the sum over sixteen lanes' row, in every lane: in pairs of lanes 1, 2, 4 and 8 apart
+template <class F>
+__device__ __forceinline__ float row16_reduce(float v, F &&op) {
+    v = op(v, dpp<0xb1>(v));      // quad_perm [1, 0, 3, 2]
+    v = op(v, dpp<0x4e>(v));      // quad_perm [2, 3, 0, 1]
+    v = op(v, dpp<0x141>(v));     // row_half_mirror
+    return op(v, dpp<0x140>(v));  // row_mirror
+}
+__device__ __forceinline__ float row16_sum(float v) { return row16_reduce(v, add2); }
+
 // op over all 64 lanes, in every lane: in pairs of lanes 1, 2, 4, 8, 16 and 32 apart
 template <class F>
 __device__ __forceinline__ float wave_reduce(float v, F &&op) {
-    v = op(v, dpp<0xb1>(v));   // quad_perm [1, 0, 3, 2]
-    v = op(v, dpp<0x4e>(v));   // quad_perm [2, 3, 0, 1]
-    v = op(v, dpp<0x141>(v));  // row_half_mirror
-    v = op(v, dpp<0x140>(v));  // row_mirror
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return op(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    return half_pair(row_pair(row16_reduce(v, op), op), op);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-    return wave_reduce(v, [](float a, float b) { return a + b; });
-}
+__device__ __forceinline__ float wave_sum(float v) { return wave_reduce(v, add2); }
 
-__device__ __forceinline__ float wave_max(float v) {
-    return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
-}
+__device__ __forceinline__ float wave_max(float v) { return wave_reduce(v, fmaxf); }
 
 constexpr float LOG2E = 1.44269504088896340736f;
 

@@ -41,7 +41,7 @@ __device__ __forceinline__ int norm_split(float (&xv)[8][8], const float *__rest
     for (int ks = 0; ks < 8; ks++)
 #pragma unroll
         for (int t = 0; t < 8; t++) sum += xv[ks][t];
-    sum += __shfl_xor(sum, 32, 64);
+    sum = half_sum(sum);
     const float mean = sum / (float)E;
     float sq = 0.0f;
 #pragma unroll
@@ -51,7 +51,7 @@ __device__ __forceinline__ int norm_split(float (&xv)[8][8], const float *__rest
             const float dv = xv[ks][t] - mean;
             sq += dv * dv;
         }
-    sq += __shfl_xor(sq, 32, 64);
+    sq = half_sum(sq);
     const float inv = 1.0f / sqrtf(sq / (float)E + 1e-5f);
     float xmax = 0.0f;
 #pragma unroll
@@ -68,7 +68,7 @@ __device__ __forceinline__ int norm_split(float (&xv)[8][8], const float *__rest
             xmax = fmaxf(xmax, fabsf(xv[ks][t]));
         }
     }
-    xmax = fmaxf(xmax, __shfl_xor(xmax, 32, 64));
+    xmax = half_max(xmax);
     const int sx = shift_for_max(xmax);
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) split8(xv[ks], ldexpf(1.0f, sx), xh[ks], xl[ks]);
@@ -153,7 +153,7 @@ __device__ __forceinline__ void ff128_rows(float (&xv)[8][8], bool live, float *
     };
     // a half of the hidden layer, activated, scaled by its own power of two and split into hh8 / hl8
     auto split_half = [&](floatx16 (&a)[4], float mx, int half) {
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = half_max(mx);
         const int sh = shift_for_max(mx);
 #pragma unroll
         for (int T = 0; T < 4; T++)

@@ -147,8 +147,7 @@ __global__ __launch_bounds__(256) void k_gemm_skinny(int M, int N, int K, const 
             *reinterpret_cast<float4 *>(xw + k) = v;
             sum += (v.x + v.y) + (v.z + v.w);
         }
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1) sum += __shfl_xor(sum, o, 64);
+        sum = row16_sum(sum);
         const float mean = sum / (float)K;
         float sq = 0.0f;
         for (int k = 4 * cc; k < K; k += 64) {
@@ -156,8 +155,7 @@ __global__ __launch_bounds__(256) void k_gemm_skinny(int M, int N, int K, const 
             const float d0 = v.x - mean, d1 = v.y - mean, d2 = v.z - mean, d3 = v.w - mean;
             sq += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
         }
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1) sq += __shfl_xor(sq, o, 64);
+        sq = row16_sum(sq);
         const float inv = 1.0f / sqrtf(sq / (float)K + 1e-5f);
         for (int k = 4 * cc; k < K; k += 64) {
             const float4 v = *reinterpret_cast<const float4 *>(xw + k);

@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(int M, int N, int K, cons
         for (int ks = 0; ks < 8; ks++)
 #pragma unroll
             for (int t = 0; t < 8; t++) xmax = fmaxf(xmax, fabsf(xv[ks][t]));
-        xmax = fmaxf(xmax, __shfl_xor(xmax, 32, 64));
+        xmax = half_max(xmax);
         const int e = shift_for_max(xmax);
         if (k0 > 0) {
             const float r = ldexpf(1.0f, e - eprev);
@@ -152,7 +152,7 @@ __device__ __forceinline__ void qmlp64_lane(const float (&xv)[4][8], int r32, in
     for (int ks = 0; ks < 4; ks++)
 #pragma unroll
         for (int t = 0; t < 8; t++) xmax = fmaxf(xmax, fabsf(xv[ks][t]));
-    xmax = fmaxf(xmax, __shfl_xor(xmax, 32, 64));
+    xmax = half_max(xmax);
     const int sx = shift_for_max(xmax);
     halfx8 xh[4], xl[4];
 #pragma unroll
@@ -184,7 +184,7 @@ __device__ __forceinline__ void qmlp64_lane(const float (&xv)[4][8], int r32, in
                 hmax = fmaxf(hmax, fabsf(hv));
             }
         }
-    hmax = fmaxf(hmax, __shfl_xor(hmax, 32, 64));
+    hmax = half_max(hmax);
     const int sh = shift_for_max(hmax);
     halfx8 hh8[4], hl8[4];
 #pragma unroll
@@ -292,7 +292,7 @@ __device__ __forceinline__ void qmlp64_tile(const float *qt, int ldq, float *hs,
         for (int ks = 0; ks < 4; ks++)
 #pragma unroll
             for (int t = 0; t < 8; t++) xmax = fmaxf(xmax, fabsf(xv[ks][t]));
-        xmax = fmaxf(xmax, __shfl_xor(xmax, 32, 64));
+        xmax = half_max(xmax);
         const int sx = shift_for_max(xmax);
         floatx16 acc;
 #pragma unroll
@@ -332,7 +332,7 @@ __device__ __forceinline__ void qmlp64_tile(const float *qt, int ldq, float *hs,
         for (int ks = 0; ks < 4; ks++)
 #pragma unroll
             for (int t = 0; t < 8; t++) hmax = fmaxf(hmax, fabsf(hv[ks][t]));
-        hmax = fmaxf(hmax, __shfl_xor(hmax, 32, 64));
+        hmax = half_max(hmax);
         const int sh = shift_for_max(hmax);
         floatx16 acc;
 #pragma unroll
@@ -478,7 +478,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_gemm_splitk4(int M, int N, int K,
             for (int ks = 0; ks < CW / 16; ks++)
 #pragma unroll
                 for (int t = 0; t < 8; t++) sum += xv[ks][t];
-            sum += __shfl_xor(sum, 32, 64);
+            sum = half_sum(sum);
             if (g == 0) rsum[wave][r32] = sum;
             __syncthreads();
             const float mean = row_total() / (float)K;
@@ -490,7 +490,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_gemm_splitk4(int M, int N, int K,
                     const float dv = xv[ks][t] - mean;
                     sq += dv * dv;
                 }
-            sq += __shfl_xor(sq, 32, 64);
+            sq = half_sum(sq);
             __syncthreads();
             if (g == 0) rsum[wave][r32] = sq;
             __syncthreads();
@@ -513,7 +513,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_gemm_splitk4(int M, int N, int K,
         for (int ks = 0; ks < CW / 16; ks++)
 #pragma unroll
             for (int t = 0; t < 8; t++) xmax = fmaxf(xmax, fabsf(xv[ks][t]));
-        xmax = fmaxf(xmax, __shfl_xor(xmax, 32, 64));
+        xmax = half_max(xmax);
         const int e = shift_for_max(xmax);
         if (k0 > wave * kq) {
             const float r = ldexpf(1.0f, e - eprev);
@@ -740,7 +740,7 @@ __global__ __launch_bounds__(512) void k_dense_few(int M, const float *__restric
         for (int j = 0; j < NST; j++)
 #pragma unroll
             for (int t = 0; t < 8; t++) sum += xv[j][t];
-        sum += __shfl_xor(sum, 32, 64);
+        sum = half_sum(sum);
         if (g == 0) rsum[wave][r32] = sum;
         __syncthreads();
         float tot = 0.0f;
@@ -755,7 +755,7 @@ __global__ __launch_bounds__(512) void k_dense_few(int M, const float *__restric
                 const float dv = xv[j][t] - mean;
                 sq += dv * dv;
             }
-        sq += __shfl_xor(sq, 32, 64);
+        sq = half_sum(sq);
         __syncthreads();
         if (g == 0) rsum[wave][r32] = sq;
         __syncthreads();
@@ -776,7 +776,7 @@ __global__ __launch_bounds__(512) void k_dense_few(int M, const float *__restric
     for (int j = 0; j < NST; j++)
 #pragma unroll
         for (int t = 0; t < 8; t++) xmax = fmaxf(xmax, fabsf(xv[j][t]));
-    xmax = fmaxf(xmax, __shfl_xor(xmax, 32, 64));
+    xmax = half_max(xmax);
     const int e = shift_for_max(xmax);
     const float f = ldexpf(1.0f, e);
     floatx16 acc[TN];
@@ -994,9 +994,10 @@ __global__ __launch_bounds__(1024) void k_query_rows(int M, const float *__restr
     __syncthreads();
     // the projection: column c, K slice sl; the slice sums over the 16 lanes of the column
     auto sum16 = [](float v) {
-#pragma unroll
-        for (int m = 8; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-        return v;
+        v += dpp<0x128>(v);  // row_ror:8, then 4, 2 and 1
+        v += dpp<0x124>(v);
+        v += dpp<0x122>(v);
+        return v + dpp<0x121>(v);
     };
 #pragma unroll
     for (int r = 0; r < QROWS; r++) {

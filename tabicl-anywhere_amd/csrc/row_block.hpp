@@ -158,7 +158,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
         for (int ks = 0; ks < 8; ks++)
 #pragma unroll
             for (int t = 0; t < 8; t++) sum += xv[ks][t];
-        sum += __shfl_xor(sum, 32, 64);
+        sum = half_sum(sum);
         const float mean = sum / 128.0f;
         float sq = 0.0f;
 #pragma unroll
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
                 const float dv = xv[ks][t] - mean;
                 sq += dv * dv;
             }
-        sq += __shfl_xor(sq, 32, 64);
+        sq = half_sum(sq);
         const float inv = 1.0f / sqrtf(sq / 128.0f + 1e-5f);
 #pragma unroll
         for (int ks = 0; ks < 8; ks++) {
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
     for (int ks = 0; ks < 8; ks++)
 #pragma unroll
         for (int t = 0; t < 8; t++) xmax = fmaxf(xmax, fabsf(xv[ks][t]));
-    xmax = fmaxf(xmax, __shfl_xor(xmax, 32, 64));
+    xmax = half_max(xmax);
     const int sx = shift_for_max(xmax);
 
     // query projection (accumulator v of tile T: head 2 T + v / 8, coordinate 8 g + v % 8), bias, rotation, 1 / 4
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
         for (int T4 = 0; T4 < 4; T4++)
 #pragma unroll
             for (int v = 0; v < 16; v++) qmax = fmaxf(qmax, fabsf(qa[T4][v]));
-        sq = shift_for_max(fmaxf(qmax, __shfl_xor(qmax, 32, 64)));
+        sq = shift_for_max(half_max(qmax));
 #pragma unroll
         for (int h = 0; h < 8; h++) {
             float qv[8];
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
         for (int h = 0; h < 8; h++)
 #pragma unroll
             for (int t = 0; t < 8; t++) omax = fmaxf(omax, fabsf(ov[h][t]));
-        so = shift_for_max(fmaxf(omax, __shfl_xor(omax, 32, 64)));
+        so = shift_for_max(half_max(omax));
         halfx8 oh[8], ol[8];
 #pragma unroll
         for (int h = 0; h < 8; h++) split8(ov[h], ldexpf(1.0f, so), oh[h], ol[h]);

@@ -159,8 +159,8 @@ __global__ __launch_bounds__(256) void k_cell_attn16(int n, size_t sr, size_t sg
     for (int kt = 0; kt < NT; kt++)
 #pragma unroll
         for (int v = 0; v < 4; v++) mx = fmaxf(mx, sacc[kt][v]);
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = row_max(mx);
+    mx = half_max(mx);
     float l = 0.0f;
 #pragma unroll
     for (int kt = 0; kt < NT; kt++)
@@ -169,8 +169,8 @@ __global__ __launch_bounds__(256) void k_cell_attn16(int n, size_t sr, size_t sg
             sacc[kt][v] = fast_exp(sacc[kt][v] - mx);
             l += sacc[kt][v];
         }
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = row_sum(l);
+    l = half_sum(l);
     floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int kt = 0; kt < NT; kt++) {
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256) void k_cell_attn_x3(int n, size_t sr, size_t s
     float qmax = 0.0f;
 #pragma unroll
     for (int k = 0; k < 8; k++) qmax = fmaxf(qmax, fabsf(qv[k]));
-    qmax = fmaxf(qmax, __shfl_xor(qmax, 32, 64));
+    qmax = half_max(qmax);
     const int sq = shift_for_max(qmax);
     halfx8 qh, ql;
     split8(qv, ldexpf(1.0f, sq), qh, ql);
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(256) void k_cell_attn_x3(int n, size_t sr, size_t s
 #pragma unroll
         for (int v = 0; v < 16; v++) mx = fmaxf(mx, sc[kt][v]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = half_max(mx);
     const float off = 12.0f - mx * to_log2;
     float l = 0.0f;
     halfx8 ph[8], pl[8];
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(256) void k_cell_attn_x3(int n, size_t sr, size_t s
             }
             split8(p, 1.0f, ph[2 * kt + hh], pl[2 * kt + hh]);
         }
-    l += __shfl_xor(l, 32, 64);
+    l = half_sum(l);
     floatx16 o;
 #pragma unroll
     for (int v = 0; v < 16; v++) o[v] = 0.0f;
@@ -647,7 +647,7 @@ __global__ __launch_bounds__(256) void k_row_attn_x3(int n, int T, int nq_tok, i
         float qmax = 0.0f;
 #pragma unroll
         for (int k = 0; k < 8; k++) qmax = fmaxf(qmax, fabsf(qv[k]));
-        qmax = fmaxf(qmax, __shfl_xor(qmax, 32, 64));
+        qmax = half_max(qmax);
         const int sq = shift_for_max(qmax);
         halfx8 qh, ql;
         split8(qv, ldexpf(1.0f, sq), qh, ql);
@@ -672,7 +672,7 @@ __global__ __launch_bounds__(256) void k_row_attn_x3(int n, int T, int nq_tok, i
 #pragma unroll
             for (int v = 0; v < 16; v++) mx = fmaxf(mx, sc[kt][v]);
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = half_max(mx);
         const float off = 12.0f - mx * to_log2;
         float l = 0.0f;
         // O^T = V^T P^T over the 16-key steps st = 2 kt + hh: A rows 0..15 the coordinates, 16..31 zero
@@ -701,7 +701,7 @@ __global__ __launch_bounds__(256) void k_row_attn_x3(int n, int T, int nq_tok, i
             }
             o = mfma16x3(ah, al, ph, pl, o);
         }
-        l += __shfl_xor(l, 32, 64);
+        l = half_sum(l);
         if (!live) continue;
         // accumulator v < 8 holds coordinate 8 (v / 4) + 4 g + v % 4 of this lane's query
         const float f = ldexpf(1.0f, -sv) / l;
