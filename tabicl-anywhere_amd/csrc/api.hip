@@ -1450,7 +1450,7 @@ static void fit_represent_on(tah_dev *dev, const tah_weights *w, const float *x,
         const ColumnBufs cb = column_bufs(w, rows, g, loans);
         float *plain = digits > 1 ? loans.take<float>(M * e) : nullptr;
         float *sum = digits > 1 ? loans.take<float>(M * e) : nullptr;
-        fit_cells(s, w, xd, rows, features, g0, g, cells);
+        fit_cells(s, w, xd, rows, features, g0, g, cells, digits == 1 ? yd : nullptr);
         if (digits > 1) {
             TAH_HIP(hipMemcpyAsync(plain, cells, M * e * sizeof(float), hipMemcpyDeviceToDevice, s));
             TAH_HIP(hipMemsetAsync(sum, 0, M * e * sizeof(float), s));
@@ -1459,7 +1459,7 @@ static void fit_represent_on(tah_dev *dev, const tah_weights *w, const float *x,
             if (dg > 0) TAH_HIP(hipMemcpyAsync(cells, plain, M * e * sizeof(float), hipMemcpyDeviceToDevice, s));
             int divisor = 1;
             for (int k = dg + 1; k < digits; k++) divisor *= bases[k];
-            add_y_cells(s, w, yd, rows, g, digits, divisor, bases[dg], cells);
+            if (digits > 1) add_y_cells(s, w, yd, rows, g, digits, divisor, bases[dg], cells);
             column_blocks(s, w, cells, rows, g, indq, col_kv, gstride, (size_t)dg * nb * per, g0, cb);
             if (digits > 1) add_to(s, M * e, cells, sum);
         }

@@ -330,7 +330,8 @@ void column_block(hipStream_t s, const tah_weights *w, const DevBlock &b, float 
                   float *mid, const uint8_t *ready = nullptr);
 
 // The column stage of a fit (fit_stages.hip).
-void fit_cells(hipStream_t s, const tah_weights *w, const float *x, int rows, int features, int g0, int gb, float *cells);
+void fit_cells(hipStream_t s, const tah_weights *w, const float *x, int rows, int features, int g0, int gb, float *cells,
+               const float *y);
 void add_y_rows(hipStream_t s, const tah_weights *w, const float *y, int rows, float *h);
 void add_y_cells(hipStream_t s, const tah_weights *w, const float *y, int rows, int gb, int digits, int divisor, int base,
                  float *cells);

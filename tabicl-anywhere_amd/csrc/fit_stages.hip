@@ -17,29 +17,61 @@ namespace tah {
 
 static dim3 blocks_of(size_t count) { return dim3((unsigned)((count + 255) / 256)); }
 
-// cells [gb][rows][e] of feature groups g0.. through the input layer.
-__global__ __launch_bounds__(256) void k_fit_cells(int rows, int features, int g0, int gb, int group, int e,
+// cells [gb][rows][e] of feature groups g0.. through the input layer, with y (one label digit) its target's embedding
+// added as k_add_y adds it. Bound by the cells' way to memory: four coordinates a thread for FIT_ROWS rows of group
+// blockIdx.y, G = group's weights in registers (G = 0: any group size, read again for each row). 1,000,000 cells: 680 us
+// with a float a thread and 400 for the embedding's pass, 592 with four floats and their weights read for every cell.
+constexpr int FIT_ROWS = 64;
+template <int G>
+__global__ __launch_bounds__(256) void k_fit_cells(int rows, int features, int g0, int group, int e,
                                                     const float *__restrict__ x, const float *__restrict__ in_w,
-                                                    const float *__restrict__ in_b, float *__restrict__ cells) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)gb * rows * e) return;
-    const int o = (int)(i % e);
-    const size_t r = (i / e) % rows;
-    const int g = g0 + (int)(i / ((size_t)e * rows));
-    const float *xr = x + r * features;
-    float vals[8];
-    bool missing = true;
-    for (int k = 0; k < group; k++) {
-        vals[k] = xr[(g + (1 << k)) % features];
-        missing = missing && vals[k] == -100.0f;
+                                                    const float *__restrict__ in_b, const float *__restrict__ y,
+                                                    int max_classes, const float *__restrict__ table,
+                                                    float *__restrict__ cells) {
+    const int n = G ? G : group, e4 = e / 4, wide = min(e4, 256), side = 256 / wide;  // rows side by side
+    const int rl = (int)threadIdx.x / wide, g = g0 + (int)blockIdx.y;
+    if (rl >= side) return;
+    const int r1 = min(rows, ((int)blockIdx.x + 1) * FIT_ROWS);
+    int from[8];
+#pragma unroll
+    for (int k = 0; k < (G ? G : 8); k++) from[k] = k < n ? (g + (1 << k)) % features : 0;
+    for (int o = 4 * ((int)threadIdx.x - rl * wide); o < e; o += 4 * wide) {
+        float w[4][G ? G : 1], b[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            b[c] = in_b[o + c];
+#pragma unroll
+            for (int k = 0; k < G; k++) w[c][k] = in_w[(o + c) * G + k];
+        }
+        for (int r = blockIdx.x * FIT_ROWS + rl; r < r1; r += side) {
+            const float *xr = x + (size_t)r * features;
+            float vals[8];
+            bool missing = true;
+#pragma unroll
+            for (int k = 0; k < (G ? G : 8); k++)
+                if (k < n) {
+                    vals[k] = xr[from[k]];
+                    missing = missing && vals[k] == -100.0f;
+                }
+            float out[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                float s = 0.0f;
+#pragma unroll
+                for (int k = 0; k < (G ? G : 8); k++)
+                    if (k < n) s += (G ? w[c][G ? k : 0] : in_w[(o + c) * group + k]) * vals[k];
+                out[c] = missing ? -100.0f : s + b[c];
+            }
+            if (y) {
+                const float yr = y[r];
+                const float *t = max_classes > 0 ? table + (size_t)(int)yr * e : table;
+#pragma unroll
+                for (int c = 0; c < 4; c++) out[c] += max_classes > 0 ? t[o + c] : t[o + c] * yr + t[e + o + c];
+            }
+            *reinterpret_cast<float4 *>(cells + ((size_t)blockIdx.y * rows + r) * e + o) =
+                make_float4(out[0], out[1], out[2], out[3]);
+        }
     }
-    if (missing) {
-        cells[i] = -100.0f;
-        return;
-    }
-    float s = 0.0f;
-    for (int k = 0; k < group; k++) s += in_w[o * group + k] * vals[k];
-    cells[i] = s + in_b[o];
 }
 
 // cells [gb][rows][e] += the target's embedding (Model::add_y, src/model.rs:188-200) of digit `(y / divisor) % base`
@@ -170,7 +202,7 @@ __global__ __launch_bounds__(256, 3) void k_ind_attn16(int gb, int rows, int ind
     load8(indq + (size_t)(live ? qi : 0) * e + h * 16 + 8 * g, qv);
 #pragma unroll
     for (int t = 0; t < 8; t++) qmax = fmaxf(qmax, fabsf(qv[t]));
-    const int sq = shift_for_max(fmaxf(qmax, __shfl_xor(qmax, 32, 64)));
+    const int sq = shift_for_max(half_max(qmax));
     halfx8 qh, ql;
     split8(qv, ldexpf(1.0f, sq), qh, ql);
     stage_max(0, st0);
@@ -314,11 +346,20 @@ __global__ __launch_bounds__(256) void k_regroup(int rows, int g, int e, const f
 }
 
 // ---- launchers ---------------------------------------------------------------------------------------------
-void fit_cells(hipStream_t s, const tah_weights *w, const float *x, int rows, int features, int g0, int gb, float *cells) {
+void fit_cells(hipStream_t s, const tah_weights *w, const float *x, int rows, int features, int g0, int gb, float *cells,
+               const float *y) {
     if (w->group > 8 || w->group < 1) throw ArgError{"column stage: feature group size must be 1..8"};
-    const size_t count = (size_t)gb * rows * w->e;
-    hipLaunchKernelGGL(k_fit_cells, blocks_of(count), dim3(256), 0, s, rows, features, g0, gb, w->group, w->e, x, w->in_w,
-                       w->in_b, cells);
+    if (w->e % 4) throw ArgError{"column stage: embedding width must be a multiple of 4"};
+    for (int k = 0; k < gb; k += 65535) {  // a launch's groups
+        const dim3 grid((rows + FIT_ROWS - 1) / FIT_ROWS, std::min(gb - k, 65535));
+        float *at = cells + (size_t)k * rows * w->e;
+        if (w->group == 3)
+            hipLaunchKernelGGL(k_fit_cells<3>, grid, dim3(256), 0, s, rows, features, g0 + k, 3, w->e, x, w->in_w, w->in_b, y,
+                               w->max_classes, w->col_y, at);
+        else
+            hipLaunchKernelGGL(k_fit_cells<0>, grid, dim3(256), 0, s, rows, features, g0 + k, w->group, w->e, x, w->in_w,
+                               w->in_b, y, w->max_classes, w->col_y, at);
+    }
     TAH_LAUNCHED();
 }
 
