@@ -113,19 +113,28 @@ def query(block, scale: np.ndarray, x: np.ndarray) -> np.ndarray:
     return (qh * (scale.reshape(block.heads, hd) * (F(1.0) + tanh1(mm)))).reshape(q.shape).astype(F)
 
 
-def query_scale(block, n: int) -> np.ndarray:
-    """`Block::query_scale` (`src/nn.rs:97-107`): what every query of the block is multiplied by with n keys."""
-    inv = F(1.0) / np.sqrt(F(block.hd))
-    if block.ss_hidden == 0:
-        return np.full(block.d, inv, F)
+def query_scales(blocks, n: int) -> np.ndarray:
+    """`Block::query_scale` (`src/nn.rs:97-107`) of each block, [blocks][d]: what its queries are multiplied by with n
+    keys. The blocks' hidden units go through GELU together, and each row's sum runs left to right in float32, as the
+    reference's matvec rows: the products' columns as contiguous rows, summed row after row."""
+    out = np.empty((len(blocks), blocks[0].d), F)
+    inv = F(1.0) / np.sqrt(F(blocks[0].hd))
+    if blocks[0].ss_hidden == 0:
+        out[:] = inv
+        return out
     logn = np.log(F(max(n, 1)))
-    hid = gelu(block.t["b0w"] * logn + block.t["b0b"])
-    w2 = block.t["b2w"].reshape(block.d, block.ss_hidden)
-    # each row's sum left to right in float32, as the reference's matvec rows: the products' columns as contiguous rows,
-    # summed row after row (accumulating along each row took 0.25 ms a block, as long as the card's work on a small layer)
-    s = np.add.reduce(np.ascontiguousarray(w2.T) * hid[:, None], axis=0, dtype=F)
-    out = (s + block.t["b2b"]).astype(F)
-    return (out * inv).astype(F)
+    hid = gelu(np.stack([b.t["b0w"] for b in blocks]) * logn + np.stack([b.t["b0b"] for b in blocks]))
+    prod = np.empty((blocks[0].ss_hidden, blocks[0].d), F)
+    for i, b in enumerate(blocks):
+        np.multiply(b.t["b2w"].reshape(b.d, b.ss_hidden).T, hid[i][:, None], out=prod)
+        np.add.reduce(prod, axis=0, dtype=F, out=out[i])
+        out[i] = (out[i] + b.t["b2b"]) * inv
+    return out
+
+
+def query_scale(block, n: int) -> np.ndarray:
+    """One block's `query_scales`."""
+    return query_scales([block], n)[0]
 
 
 def input_cells(m, x: np.ndarray, y: np.ndarray, g0: int, gn: int) -> np.ndarray:
@@ -186,7 +195,7 @@ def fit_raw_hooks(gpu, weights, x, y, classes: int, chunk: int = 256, kv_format:
     for node in plan.nodes:
         h = reps.copy() if node.rows is None else reps[np.asarray(node.rows, np.int64)]
         m.add_y(m.t["icl_y"], np.asarray(node.y, F), h)
-        scales = np.stack([query_scale(b, rows if node.rows is None else len(node.rows)) for b in m.icl]).astype(F)
+        scales = query_scales(m.icl, rows if node.rows is None else len(node.rows))
         layers = []
         gpu.in_context_fit(weights, h, scales, kv_format, chunk, lambda l, rec: layers.append(copy_records(rec)))
         fitted.scales.append(scales)
@@ -255,11 +264,11 @@ def fit_raw(gpu, weights, x, y, classes: int, chunk: int = 256, kv_format: int =
     rows, features = x.shape
     chunk = max(int(chunk), 8)
     plan = Plan.new(m.max_classes, y, classes)
-    ind_scales = np.stack([query_scale(b, rows) for b in m.col_a1]).astype(F)
+    ind_scales = query_scales(m.col_a1, rows)
     if len(plan.nodes) == 1 and len(plan.bases) == 1 and (m.max_classes == 0 or (y.size and y.min() >= 0 and
                                                                               y.max() < m.max_classes)):
         # one problem over the whole table: the representations stay on the card
-        scales = np.stack([query_scale(b, rows) for b in m.icl]).astype(F)
+        scales = query_scales(m.icl, rows)
         layers = []
         col_kv = gpu.fit(weights, x, y, plan.bases[0], ind_scales, scales, kv_format, chunk,
                          lambda l, rec: layers.append(copy_records(rec)))
@@ -275,7 +284,7 @@ def fit_raw(gpu, weights, x, y, classes: int, chunk: int = 256, kv_format: int =
         else:
             h = reps.copy()
         m.add_y(m.t["icl_y"], np.asarray(node.y, F), h)
-        scales = np.stack([query_scale(b, n_rows) for b in m.icl]).astype(F)
+        scales = query_scales(m.icl, n_rows)
         layers = []
         gpu.in_context_fit(weights, h, scales, kv_format, chunk, lambda l, rec: layers.append(copy_records(rec)))
         fitted.scales.append(scales)
