@@ -135,7 +135,8 @@ __device__ __forceinline__ float fast_exp(float x) { return exp2_hw(x * LOG2E); 
 // elements above 2^-17 of the largest.
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef __fp16 fp16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
 // Reinterpret whole vectors only: this compiler turns __builtin_bit_cast(T, v[i]) of a vector element into element 0
 // for every i (copy the element into a scalar first).
 
@@ -164,19 +165,25 @@ __device__ __forceinline__ floatx16 mfma16x3(halfx8 ah, halfx8 al, halfx8 bh, ha
     return mfma16(al, bh, c);
 }
 
-__device__ __forceinline__ uint32_t bits(fp16x2 h) { return __builtin_bit_cast(uint32_t, h); }
+// two floats as fp16, each rounded to the nearest (v_cvt_pk_f16_f32)
+__device__ __forceinline__ uint32_t half_pair_bits(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{a, b}), halfx2));
+}
 
-// hi/lo fp16 halves of two floats, hi rounded toward zero (the residual x - hi is exact in f32). The residuals come
+// hi/lo fp16 halves of two floats, both rounded to the nearest (the residual x - hi is exact in f32): with the low half's
+// sign 23 bits, the dropped lo lo products at most 2^-22 of their terms and of either sign. Cut off instead, the halves hold
+// 22 bits and the dropped products all have their terms' sign (a fit's first layer, 3,000 x 100, from 64 bits: 3.06e-7 cut off,
+// 2.31e-7 rounded, 2.89e-7 with the column and wide-row attention on f32 matrix instructions). The residuals come
 // from v_fma_mix_f32 reading each fp16 half of hi directly (x + (-1) hi, one instruction each, where a conversion
 // back to f32 and a subtraction would take two). The last writer of lo stays an ordinary instruction (the packing
 // conversion): the compiler inserts the wait states a matrix instruction needs after it, which it cannot do after
 // inline assembly (v_fma_mix{lo,hi}_f16 writing lo directly gave wrong products).
 __device__ __forceinline__ void split2(float a, float b, uint32_t &hi, uint32_t &lo) {
-    hi = bits(__builtin_amdgcn_cvt_pkrtz(a, b));
+    hi = half_pair_bits(a, b);
     float ra, rb;
     asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(ra) : "v"(hi), "v"(a));
     asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rb) : "v"(hi), "v"(b));
-    lo = bits(__builtin_amdgcn_cvt_pkrtz(ra, rb));
+    lo = half_pair_bits(ra, rb);
 }
 
 // The floats hi + lo of two split values (hi: their two fp16 high halves, lo: their low halves), exact, one
