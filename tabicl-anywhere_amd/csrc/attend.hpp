@@ -36,6 +36,16 @@ __device__ __forceinline__ void pad_rows(uint8_t *pad, int tid, int per, int T) 
     }
 }
 
+// The shifts of eight heads' queries, four to a register (held through all heads, where a register a head meant spills).
+// From -128 to 127 (14 - 128 is the least there is).
+struct HeadShifts {
+    int w[2] = {0, 0};
+    __device__ __forceinline__ void set(int h, int shift) { w[h >> 2] |= (shift & 255) << (8 * (h & 3)); }
+    // behind the last set: the compiler would otherwise keep the eight shifts it packed
+    __device__ __forceinline__ void pack() { asm volatile("" : "+v"(w[0]), "+v"(w[1])); }
+    __device__ __forceinline__ int get(int h) const { return (int)(int8_t)(w[h >> 2] >> (8 * (h & 3))); }
+};
+
 template <int NT>
 __device__ __forceinline__ floatx16 score_tile(const uint8_t *kb, int j, halfx8 qh, halfx8 ql) {
     const halfx8 ah = *reinterpret_cast<const halfx8 *>(kb + 512 * j);

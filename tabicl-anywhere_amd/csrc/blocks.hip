@@ -449,8 +449,8 @@ __device__ __forceinline__ void in_cell8(const InCells &ic, const float (&vals)[
 // (cell (r, g) at row r sr + g sg of cells), lane l cell l % 32, as the B operand of every product:
 //  * query projection H^T = Wq X^T as in k_rows128 (its accumulators hold, for each head, eight consecutive query
 //    coordinates 8 (l / 32) + 0..7: the B operand of the head's S^T = K Q^T);
-//  * the queries are split for all heads at one power of two a cell; per head the attention of attend.hpp over the
-//    group's image, the next head's scores formed between this head's weights;
+//  * the queries are split, each head's at its own power of two; per head the attention of attend.hpp over the group's
+//    image, the next head's scores formed between this head's weights;
 //  * the heads' outputs, split at the least of the heads' value scales (an output is at most its values' largest
 //    magnitude), take the queries' registers, and the output projection runs once behind all heads;
 //  * LDS (72 KB, two workgroups a compute unit): the query weights (64 KB) first, then four head images, two heads
@@ -581,24 +581,22 @@ __global__ __launch_bounds__(256, 2) void k_cell_block(int n, size_t sr, size_t 
                 for (int t = 0; t < 8; t++) qa[T][8 * hh + t] = (qa[T][8 * hh + t] * u + bv[t]) * cv[t];
             }
     }
-    // the queries split at one power of two for all heads (head h: coordinates 8 g + t of tile h / 2)
+    // the queries, each head's split at its own power of two (head h: coordinates 8 g + t of tile h / 2)
     halfx8 qh[8], ql[8];
-    int sq;
-    {
-        float qmax = 0.0f;
+    HeadShifts sq;
 #pragma unroll
-        for (int T = 0; T < 4; T++)
+    for (int h = 0; h < 8; h++) {
+        float qv[8], qmax = 0.0f;
 #pragma unroll
-            for (int v = 0; v < 16; v++) qmax = fmaxf(qmax, fabsf(qa[T][v]));
-        sq = shift_for_max(half_max(qmax));
-#pragma unroll
-        for (int h = 0; h < 8; h++) {
-            float qv[8];
-#pragma unroll
-            for (int t = 0; t < 8; t++) qv[t] = qa[h >> 1][8 * (h & 1) + t];
-            split8(qv, ldexpf(1.0f, sq), qh[h], ql[h]);
+        for (int t = 0; t < 8; t++) {
+            qv[t] = qa[h >> 1][8 * (h & 1) + t];
+            qmax = fmaxf(qmax, fabsf(qv[t]));
         }
+        const int s = min(shift_for_max(half_max(qmax)), 127);
+        sq.set(h, s);
+        split8(qv, ldexpf(1.0f, s), qh[h], ql[h]);
     }
+    sq.pack();
     __syncthreads();  // everyone is done with the query weights
     // image h in slot h % 4, copied in two to three heads ahead; behind the last images the output projection's weights
     dma_to_lds(gimg, lds, CIMG, tid);
@@ -624,7 +622,7 @@ __global__ __launch_bounds__(256, 2) void k_cell_block(int n, size_t sr, size_t 
             dma_to_lds(gimg + (size_t)(h + 2) * CIMG, lds + ((h + 2) & 3) * CIMG, CIMG, tid);
         else if (h >= 6)
             dma_to_lds(oimg + (size_t)(h - 6) * CIMG, lds + (h - 6) * CIMG, CIMG, tid);
-        const float to_log2 = ldexpf(LOG2E, -(gsh[2 * h] + sq));
+        const float to_log2 = ldexpf(LOG2E, -(gsh[2 * h] + sq.get(h)));
         float ref;
         floatx16 o;
         attend_tiles<NT, 4, true>(sc, to_log2, lds, vb + (h & 3) * vstep, ref, o, [&](int j) {

@@ -18,7 +18,7 @@ namespace tah {
 // wavefront w owns tokens 32 (w % (W / R)) + 0..31 of row w / (W / R) of the workgroup's, lane l token l % 32, as the B
 // operand of every product (as in k_cell_block):
 //  * the query projection as in k_cell_block, its accumulators rotated in registers (a coordinate's partner for the
-//    rotation sits on lane l ^ 32) and scaled by 1 / sqrt(16), then split at one power of two a token;
+//    rotation sits on lane l ^ 32) and scaled by 1 / sqrt(16), then split, each head's at its own power of two;
 //  * per head the workgroup stages its rows' keys (rotated) and values into LDS split into fp16 halves, scaled by the
 //    head's power of two (a maximum over the row's tokens, across wavefronts through LDS): half the threads a key
 //    each, the others two coordinates of eight values. Staging runs two heads ahead, its loads three: their maxima are
@@ -237,24 +237,22 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
                 }
             }
     }
-    // the queries split at one power of two for all heads, as in k_cell_block
+    // the queries, each head's split at its own power of two, as in k_cell_block
     halfx8 qh[8], ql[8];
-    int sq;
-    {
-        float qmax = 0.0f;
+    HeadShifts sq;
 #pragma unroll
-        for (int T4 = 0; T4 < 4; T4++)
+    for (int h = 0; h < 8; h++) {
+        float qv[8], qmax = 0.0f;
 #pragma unroll
-            for (int v = 0; v < 16; v++) qmax = fmaxf(qmax, fabsf(qa[T4][v]));
-        sq = shift_for_max(half_max(qmax));
-#pragma unroll
-        for (int h = 0; h < 8; h++) {
-            float qv[8];
-#pragma unroll
-            for (int t = 0; t < 8; t++) qv[t] = qa[h >> 1][8 * (h & 1) + t];
-            split8(qv, ldexpf(1.0f, sq), qh[h], ql[h]);
+        for (int t = 0; t < 8; t++) {
+            qv[t] = qa[h >> 1][8 * (h & 1) + t];
+            qmax = fmaxf(qmax, fabsf(qv[t]));
         }
+        const int s = min(shift_for_max(half_max(qmax)), 127);
+        sq.set(h, s);
+        split8(qv, ldexpf(1.0f, s), qh[h], ql[h]);
     }
+    sq.pack();
     __syncthreads();  // everyone is done with the query weights
     pad_rows<NT>(lds + PAD, tid, PER, T);
     stage_store(st0, 0, 0);
@@ -294,7 +292,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
             if (h == 6) dma_to_lds<THREADS>(oimg + 32768, lds + 32768, 16384, tid);
             if (h == 7) dma_to_lds<THREADS>(oimg, lds, 16384, tid);
         }
-        const float to_log2 = ldexpf(LOG2E, -(shs[buf][0][rs] + sq));
+        const float to_log2 = ldexpf(LOG2E, -(shs[buf][0][rs] + sq.get(h)));
         const int svh = shs[buf][1][rs];
         float ref;
         floatx16 o;
