@@ -46,6 +46,14 @@ struct HeadShifts {
     __device__ __forceinline__ int get(int h) const { return (int)(int8_t)(w[h >> 2] >> (8 * (h & 3))); }
 };
 
+// The output projection's sums from the input scale 2^from to 2^to (the same in every lane, to <= from).
+__device__ __forceinline__ void lower_scale(floatx16 (&acc)[4], int from, int to) {
+    if (to == from) return;
+    const float r = ldexpf(1.0f, to - from);
+#pragma unroll
+    for (int T = 0; T < 4; T++) acc[T] *= r;
+}
+
 template <int NT>
 __device__ __forceinline__ floatx16 score_tile(const uint8_t *kb, int j, halfx8 qh, halfx8 ql) {
     const halfx8 ah = *reinterpret_cast<const halfx8 *>(kb + 512 * j);

@@ -451,8 +451,9 @@ __device__ __forceinline__ void in_cell8(const InCells &ic, const float (&vals)[
 //    coordinates 8 (l / 32) + 0..7: the B operand of the head's S^T = K Q^T);
 //  * the queries are split, each head's at its own power of two; per head the attention of attend.hpp over the group's
 //    image, the next head's scores formed between this head's weights;
-//  * the heads' outputs, split at the least of the heads' value scales (an output is at most its values' largest
-//    magnitude), take the queries' registers, and the output projection runs once behind all heads;
+//  * the heads' outputs, split at the least of the value scales of the heads up to theirs (an output is at most its
+//    values' largest magnitude), take the queries' registers, and the output projection runs once behind all heads, its
+//    sums rescaled where a head's scale is lower than all before;
 //  * LDS (72 KB, two workgroups a compute unit): the query weights (64 KB) first, then four head images, two heads
 //    ahead of their use by DMA (one barrier a head), then the output projection's weights, half of them under the last
 //    two heads; behind these the rows of ones.
@@ -602,9 +603,9 @@ __global__ __launch_bounds__(256, 2) void k_cell_block(int n, size_t sr, size_t 
     dma_to_lds(gimg, lds, CIMG, tid);
     dma_to_lds(gimg + CIMG, lds + CIMG, CIMG, tid);
     dma_to_lds(gimg + 2 * CIMG, lds + 2 * CIMG, CIMG, tid);
-    int so = gsh[1];  // the projection's input scale (log2): the least of the heads' (an output is at most its values' max)
-#pragma unroll
-    for (int h = 1; h < 8; h++) so = min(so, gsh[2 * h + 1]);
+    // the projection's input scale (log2): the least of the values' of the heads up to this one (an output is at most its
+    // values' largest magnitude)
+    int so = gsh[1];
     const bool one = (r32 & 27) == 16;  // rows 16 and 20 of V^T are ones: accumulator 8 sums the weights
     const int vstep = one ? 0 : CIMG, kb = (g * NT + arow) * 16;
     const int vb = one ? PAD + 16 * g : NT * 64 + 256 * g + 16 * ((r32 & 15) ^ g);
@@ -629,6 +630,7 @@ __global__ __launch_bounds__(256, 2) void k_cell_block(int n, size_t sr, size_t 
             if (h + 1 < 8) sc[j] = score_tile<NT>(lds + ((h + 1) & 3) * CIMG + kb, j, qh[(h + 1) & 7], ql[(h + 1) & 7]);
         });
         float ov[8];
+        so = min(so, gsh[2 * h + 1]);
         const float f = ldexpf(1.0f, so - gsh[2 * h + 1]) / o[8];
 #pragma unroll
         for (int t = 0; t < 8; t++) ov[t] = o[t] * f;
@@ -640,20 +642,25 @@ __global__ __launch_bounds__(256, 2) void k_cell_block(int n, size_t sr, size_t 
     for (int T = 0; T < 4; T++)
 #pragma unroll
         for (int v = 0; v < 16; v++) acc[T][v] = 0.0f;
+    so = gsh[1];
 #pragma unroll
     for (int half = 0; half < 2; half++) {
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         if (half == 0) dma_to_lds(oimg + 32768, lds + 32768, 32768, tid);
 #pragma unroll
-        for (int c = 0; c < 4; c++)
+        for (int c = 0; c < 4; c++) {
+            const int ks = 4 * half + c, sn = min(so, gsh[2 * ks + 1]);
+            lower_scale(acc, so, sn);
+            so = sn;
 #pragma unroll
             for (int T = 0; T < 4; T++) {
-                const int ks = 4 * half + c, nn = 32 * T + arow;
+                const int nn = 32 * T + arow;
                 const halfx8 ah = *reinterpret_cast<const halfx8 *>(lds + ks * 8192 + (g * 128 + nn) * 16);
                 const halfx8 al = *reinterpret_cast<const halfx8 *>(lds + ks * 8192 + ((2 + g) * 128 + nn) * 16);
                 acc[T] = mfma16x3(ah, al, oh[ks], ol[ks], acc[T]);
             }
+        }
     }
     if (!FF && !live) return;
     // column of accumulator v of tile T: 32 T + 16 (v / 8) + 8 g + v % 8

@@ -266,7 +266,9 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
                    rs * (PER * 32 + (one ? 128 : 0));
     constexpr int NA = NTL < 4 ? NTL : 4, NB = NTL - NA;  // a head's key tiles, as one group of up to four or two
     floatx16 sc[NA];
-    float ov[8][8];
+    // the heads' outputs, split as the output projection's input at the least of the value scales of the heads up to theirs
+    halfx8 oh[8], ol[8];
+    int so[8];
 #pragma unroll
     for (int h = 0; h < 8; h++) {
         const int buf = h % 3, nbuf = (h + 1) % 3;
@@ -283,17 +285,18 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
             stage_load(h + 3, stv);
             __builtin_amdgcn_sched_barrier(0);  // the loads go out here
         }
-        // behind the last staged head the output projection's weights, 16-column steps of 8 KB: W = 8, 0..3 and 4..7 into
-        // the buffers of heads 5 and 6; W = 4, steps k at 8 KB k, 7 past the ones, 4, 5 and 0, 1 into those buffers
+        // behind the last staged head the output projection's weights, 16-column steps of 8 KB in the heads' order: W = 8,
+        // 0..3 and 4..7 into the buffers of heads 5 and 6; W = 4, 0 past the ones, 1, 2 and 3, 4 into those buffers
         if constexpr (W == 8) {
             if (h >= 6) dma_to_lds<THREADS>(oimg + (h - 6) * 32768, lds + (h == 6 ? 2 : 0) * STAGED, 32768, tid);
         } else {
-            if (h == 5) dma_to_lds<THREADS>(oimg + 57344, lds + 57344, 8192, tid);
-            if (h == 6) dma_to_lds<THREADS>(oimg + 32768, lds + 32768, 16384, tid);
-            if (h == 7) dma_to_lds<THREADS>(oimg, lds, 16384, tid);
+            if (h == 5) dma_to_lds<THREADS>(oimg, lds + 57344, 8192, tid);
+            if (h == 6) dma_to_lds<THREADS>(oimg + 8192, lds + 32768, 16384, tid);
+            if (h == 7) dma_to_lds<THREADS>(oimg + 24576, lds, 16384, tid);
         }
         const float to_log2 = ldexpf(LOG2E, -(shs[buf][0][rs] + sq.get(h)));
-        const int svh = shs[buf][1][rs];
+        const int svh = __builtin_amdgcn_readfirstlane(shs[buf][1][rs]);  // a wavefront's tokens are one row's
+        so[h] = h ? min(so[h - 1], svh) : svh;
         float ref;
         floatx16 o;
         const uint8_t *kn0 = lds + nbuf * STAGED + kb;
@@ -312,24 +315,16 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
 #pragma unroll
             for (int j = NB; j < NA; j++) ahead(j);
         }
-        const float f = ldexpf(1.0f, -svh) / o[8];
+        const float f = ldexpf(1.0f, so[h] - svh) / o[8];
+        float ov[8];
 #pragma unroll
-        for (int t = 0; t < 8; t++) ov[h][t] = o[t] * f;
+        for (int t = 0; t < 8; t++) ov[t] = o[t] * f;
+        split8(ov, 1.0f, oh[h], ol[h]);
         if (h + 3 < 8) stage_max(stv, (h + 3) % 3);
     }
-    // output projection, its input scaled by the token's power of two
+    // output projection
     floatx16 acc[4];
-    int so;
     {
-        float omax = 0.0f;
-#pragma unroll
-        for (int h = 0; h < 8; h++)
-#pragma unroll
-            for (int t = 0; t < 8; t++) omax = fmaxf(omax, fabsf(ov[h][t]));
-        so = shift_for_max(half_max(omax));
-        halfx8 oh[8], ol[8];
-#pragma unroll
-        for (int h = 0; h < 8; h++) split8(ov[h], ldexpf(1.0f, so), oh[h], ol[h]);
 #pragma unroll
         for (int T4 = 0; T4 < 4; T4++)
 #pragma unroll
@@ -337,20 +332,20 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();  // everyone is done with the staged heads; the weights copied through the last heads have landed
         if (W == 4) {
-            dma_to_lds<THREADS>(oimg + 16384, lds + 16384, 16384, tid);
-            dma_to_lds<THREADS>(oimg + 49152, lds + 49152, 8192, tid);
+            dma_to_lds<THREADS>(oimg + 40960, lds + 16384, 16384, tid);
+            dma_to_lds<THREADS>(oimg + 57344, lds + 49152, 8192, tid);
         }
-        constexpr int ORDER[8] = {4, 5, 0, 1, 7, 2, 3, 6};
+        constexpr int AT[8] = {57344, 32768, 40960, 0, 8192, 16384, 24576, 49152};  // W = 4: where each step is
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int ks = ORDER[i];
-            if (W == 4 && i == 5) {
+        for (int ks = 0; ks < 8; ks++) {
+            if (W == 4 && ks == 5) {
                 __builtin_amdgcn_s_waitcnt(0);
                 __syncthreads();  // the rest of the weights
             }
+            if (ks > 0) lower_scale(acc, so[ks - 1], so[ks]);
+            const uint8_t *ws = lds + (W == 4 ? AT[ks] : ks < 4 ? 2 * STAGED + ks * 8192 : (ks - 4) * 8192);
 #pragma unroll
             for (int T4 = 0; T4 < 4; T4++) {
-                const uint8_t *ws = lds + (W == 4 ? ks * 8192 : ks < 4 ? 2 * STAGED + ks * 8192 : (ks - 4) * 8192);
                 const int nn = 32 * T4 + arow;
                 const halfx8 ah = *reinterpret_cast<const halfx8 *>(ws + (g * 128 + nn) * 16);
                 const halfx8 al = *reinterpret_cast<const halfx8 *>(ws + ((2 + g) * 128 + nn) * 16);
@@ -359,7 +354,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_row_block(int n, int T, int keep,
         }
     }
     if (!FF && !live) return;
-    const float u = ldexpf(1.0f, -(so + oshift));
+    const float u = ldexpf(1.0f, -(so[7] + oshift));
     float xn[8][8];  // the new values as the feed-forward's input: columns 16 ks + 8 g + t
 #pragma unroll
     for (int T4 = 0; T4 < 4; T4++)

@@ -2,7 +2,8 @@
 have no part in the result, so that the other heads must come out as if it were not there. Against the oracle at the
 stages' raw-score tolerance, 5e-5; a scale shared with the large head would leave the others eight bits.
 
-Queries: head 0's query bias is 2^30 and its keys are zero (its weights are equal)."""
+Queries: head 0's query bias is 2^30 and its keys are zero (its weights are equal). Values: head 7's are 2^30 and the
+output projection's columns for it zero."""
 import numpy as np
 import pytest
 
@@ -33,14 +34,23 @@ def large_queries():
     return m
 
 
-@pytest.fixture(scope="module", params=["queries"])
+def large_values():
+    m = M.Model.random(M.FULL_CLASSIFIER, seed=2)
+    for b in m.col_a2 + m.row[:-1]:
+        e = b.d
+        b.t["in_b"][2 * e + 112:] = BIG
+        b.t["out_w"].reshape(e, e)[:, 112:] = 0.0
+    return m
+
+
+@pytest.fixture(scope="module", params=["queries", "values"])
 def kind(request):
     return request.param
 
 
 @pytest.fixture(scope="module")
 def model(kind):
-    return large_queries()
+    return large_queries() if kind == "queries" else large_values()
 
 
 @pytest.fixture(scope="module")
@@ -62,6 +72,8 @@ def test_column_blocks(gpu, kind, model, weights):
     col = (rng.standard_normal((features, 1, len(model.col_a2), 2, model.e, model.inds)) * 0.5).astype(np.float32)
     if kind == "queries":
         col[:, :, :, 0, :16] = 0.0
+    else:
+        col[:, :, :, 1, 112:] *= BIG
     layers = [orc.pack((rng.standard_normal(2 * model.d * rows) * 0.5).astype(np.float32), model.d, rows, abi.KV_F32)
               for _ in range(model.icl_layers)]
     scales = np.stack([orc.query_scale(b, rows) for b in model.icl])
@@ -80,7 +92,7 @@ def test_fit_columns(gpu, kind, model, weights):
     x, y = rng.standard_normal((300, 5)).astype(np.float32), rng.integers(0, 10, 300).astype(np.float32)
     got, reps = gpu.fit_represent(weights, x, y, [10], np.stack([fit.query_scale(b, 300) for b in model.col_a1]))
     want, emb = orc.fit_columns(model, x, y, [10], 256)
-    keep = np.abs(want) < 1e6
+    keep = np.abs(want) < 1e6  # all but the large head's values
     err = max(np.abs(got - want)[keep].max(), np.abs(reps - orc.fit_rows(model, emb)).max())
     say(f"large {kind}, a fit: {err:.2e}")
     assert err < TOL
