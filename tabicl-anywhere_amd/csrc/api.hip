@@ -96,14 +96,17 @@ static size_t loan_raw(size_t bytes) {
 }
 
 // Rows a call takes at a time: all n when their working memory fits the room the budget leaves, else the largest
-// halving of n that fits (rows are independent); an OutOfMemory error when not even one row fits.
+// halving of n that fits together with the shorter batch it leaves at the end (rows are independent; fewer rows may take
+// more memory, where the row stage's compact layout starts at a row count); an OutOfMemory error when not even one row
+// fits.
 template <class F>
 static int batch_rows(const tah_dev *dev, int n, F bytes_of) {
     const size_t used = busy_bytes(dev->pool);
     const size_t room = dev->pool.budget > used ? dev->pool.budget - used : 0;
+    auto fits = [&](int b) { return bytes_of(b) <= room && (n % b == 0 || bytes_of(n % b) <= room); };
     int b = std::max(n, 1);
-    while (b > 1 && bytes_of(b) > room) b = (b + 1) / 2;
-    if (bytes_of(b) > room) throw BudgetError{"graphics card: one row does not fit the working-memory budget"};
+    while (b > 1 && !fits(b)) b = (b + 1) / 2;
+    if (!fits(b)) throw BudgetError{"graphics card: one row does not fit the working-memory budget"};
     return b;
 }
 
@@ -1536,10 +1539,12 @@ static size_t columns_call_bytes(const tah_weights *w, int rows, int g) {
     return column_bufs_bytes(w, rows, g) + loan_bytes({M * e, M * e, (size_t)g * nb * 2 * e * w->inds, nb * w->inds * e});
 }
 
-// Bytes a tah_rows call borrows for n rows of `features` cells.
-static size_t rows_call_bytes(const tah_weights *w, int n, int features) {
+// Bytes a tah_rows call borrows for n rows of `features` cells; at most, for any count up to n (a caller's last batch is
+// shorter, and fewer rows may take more).
+static size_t rows_call_bytes(const tah_weights *w, int n, int features, bool any_up_to = false) {
     const size_t T = (size_t)w->cls + features, k = n;
-    return loan_bytes({k * features * w->e, k * T * w->e, k * w->d, row_stage_floats(w, n, (int)T)});
+    return loan_bytes({k * features * w->e, k * T * w->e, k * w->d,
+                       any_up_to ? row_stage_floats_up_to(w, n, (int)T) : row_stage_floats(w, n, (int)T)});
 }
 
 // The room the budget leaves now, read under the device's lock.
@@ -1568,7 +1573,11 @@ extern "C" size_t tah_column_batch(const tah_dev *dev, const tah_weights *w, int
     if (!dev || !w || rows <= 0 || w->col_a1.empty() || w->col_a2.empty() || !w->col_ind || !w->col_scale) return 0;
     // a batch's cells are one launch's rows at most
     const int cap = (int)std::min<long>(4096, std::max<long>(1, 0x7FFFFFFFL / ((long)rows * w->e)));
-    return largest_fitting(room_of(dev), cap, [&](int g) { return columns_call_bytes(w, rows, g); });
+    // every smaller count has to fit as well, and the inducing points' split sums do not only grow with the count
+    const size_t room = room_of(dev);
+    int g = 0;
+    while (g < cap && columns_call_bytes(w, rows, g + 1) <= room) g++;
+    return (size_t)g;
 }
 
 extern "C" int tah_columns(tah_dev *dev, const tah_weights *w, float *cells, int32_t rows, int32_t groups,
@@ -1603,7 +1612,7 @@ extern "C" int tah_columns(tah_dev *dev, const tah_weights *w, float *cells, int
 
 extern "C" size_t tah_row_batch(const tah_dev *dev, const tah_weights *w, int32_t features) {
     if (!dev || !w || features <= 0 || w->row.empty() || !w->cls_tokens) return 0;
-    return largest_fitting(room_of(dev), 32768, [&](int n) { return rows_call_bytes(w, n, features); });
+    return largest_fitting(room_of(dev), 32768, [&](int n) { return rows_call_bytes(w, n, features, true); });
 }
 
 extern "C" int tah_rows(tah_dev *dev, const tah_weights *w, const float *cells, int32_t n, int32_t features,

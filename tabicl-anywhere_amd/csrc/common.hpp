@@ -318,6 +318,7 @@ void column_stage_tokens(hipStream_t s, const tah_weights *w, const float *col_k
 // The first row block's keys and values of the class tokens, [cls][2 e] into out (tmp: cls e floats).
 void class_token_kv(hipStream_t s, const tah_weights *w, float *out, float *tmp);
 size_t row_stage_floats(const tah_weights *w, int n, int T);
+size_t row_stage_floats_up_to(const tah_weights *w, int n, int T);  // the most for any count of 1 to n rows
 bool row_stage_takes_kv(const tah_weights *w, int n, int T);
 float *row_stage_kv(const tah_weights *w, int n, int T, float *scratch);
 // kv_ready: the first row block's keys and values are in row_stage_kv(scratch) already (row_stage_takes_kv).

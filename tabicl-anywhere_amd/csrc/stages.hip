@@ -1084,6 +1084,17 @@ size_t row_stage_floats(const tah_weights *w, int n, int T) {
     return R * (5 * e + ff) + M * 2 * e;
 }
 
+size_t row_stage_floats_up_to(const tah_weights *w, int n, int T) {
+    const size_t here = row_stage_floats(w, n, T);
+    if (!row_stage_compact(w, n, T)) return here;
+    int lo = 0, hi = n;  // rows are compact from hi on, not up to lo
+    while (lo + 1 < hi) {
+        const int mid = lo + (hi - lo) / 2;
+        (row_stage_compact(w, mid, T) ? hi : lo) = mid;
+    }
+    return lo ? std::max(here, row_stage_floats(w, lo, T)) : here;
+}
+
 float *row_stage_kv(const tah_weights *w, int n, int T, float *scratch) {
     return scratch + (row_stage_compact(w, n, T) ? (size_t)n * w->cls : (size_t)n * T) * w->e;
 }
