@@ -92,6 +92,18 @@ __global__ __launch_bounds__(256) void k_add_y(int rows, int gb, int e, int max_
     }
 }
 
+// h [rows][d] += the in-context stage's target embedding, rounded as Model::add_y rounds it on the host (the product, the
+// sum, then the addition to h, none contracted), so that a fit in one call stores the records of the calls apart.
+__global__ __launch_bounds__(256) void k_add_y_rows(int rows, int d, int max_classes, const float *__restrict__ y,
+                                                    const float *__restrict__ table, float *__restrict__ h) {
+#pragma clang fp contract(off)
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (size_t)rows * d) return;
+    const int o = (int)(i % d);
+    const float yr = y[i / d];
+    h[i] += max_classes > 0 ? table[(size_t)(int)yr * d + o] : table[o] * yr + table[d + o];
+}
+
 __global__ __launch_bounds__(256) void k_scale_by(size_t count, const float *__restrict__ src, float f, float *__restrict__ dst) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < count) dst[i] = src[i] * f;
@@ -375,8 +387,8 @@ void add_y_cells(hipStream_t s, const tah_weights *w, const float *y, int rows, 
 
 // rows [rows][d] += the in-context stage's target embedding (Model::add_y, src/model.rs:188-200).
 void add_y_rows(hipStream_t s, const tah_weights *w, const float *y, int rows, float *h) {
-    hipLaunchKernelGGL(k_add_y, blocks_of((size_t)rows * w->d), dim3(256), 0, s, rows, 1, w->d, w->max_classes, 1, 1, 1, y,
-                       w->icl_y, h);
+    hipLaunchKernelGGL(k_add_y_rows, blocks_of((size_t)rows * w->d), dim3(256), 0, s, rows, w->d, w->max_classes, y, w->icl_y,
+                       h);
     TAH_LAUNCHED();
 }
 

@@ -74,13 +74,8 @@ def test_fit_in_one_call(gpu, kind, model, weights, rows, features, kv_format, c
     col, layers = apart(gpu, weights, x, y, base, kv_format, chunk)
     got = fit.fit_raw(gpu, weights, x, y, base, chunk, kv_format)
     assert np.array_equal(got.col_kv, col)
-
     assert len(got.layers[0]) == len(layers) == model.icl_layers
-    if kind == "clf":
-        assert all(np.array_equal(a, b) for a, b in zip(got.layers[0], layers))
-    elif kv_format == abi.KV_F32:
-        # the embedding's multiply and add are one rounding on the card, two on the host: 2^-24 of it, carried on
-        assert max(np.abs(a.view(np.float32) - b.view(np.float32)).max() for a, b in zip(got.layers[0], layers)) < TOL
+    assert all(np.array_equal(a, b) for a, b in zip(got.layers[0], layers))
 
 
 @pytest.mark.parametrize("rows,kv_format", [(300, abi.KV_I8), (1100, abi.KV_F32)])
