@@ -7,10 +7,9 @@
 #include <initializer_list>
 #include <memory>
 #include <new>
-#include <system_error>
-#include <thread>
 
 #include "common.hpp"
+#include "host_copy.hpp"
 
 using namespace tah;
 
@@ -939,31 +938,6 @@ struct SideWork {
         TAH_HIP(hipStreamWaitEvent(dev->side, dev->fork_ev, 0));
     }
 };
-
-// bytes from one host buffer to another, sliced over a few threads when large (one thread copies to pages it touches
-// for the first time at about 10 GB/s, less than the card delivers them).
-static void host_copy(uint8_t *dst, const uint8_t *src, size_t bytes) {
-    constexpr size_t SLICE = 2 << 20;
-    const size_t n = std::min<size_t>(8, bytes / SLICE);
-    if (n < 2) {
-        std::memcpy(dst, src, bytes);
-        return;
-    }
-    const size_t step = (bytes / n + 4095) & ~size_t(4095);
-    std::vector<std::thread> threads;
-    threads.reserve(n);
-    size_t at = step;  // the first slice is this thread's
-    try {
-        for (; at < bytes; at += step) {
-            const size_t k = std::min(step, bytes - at);
-            threads.emplace_back([=] { std::memcpy(dst + at, src + at, k); });
-        }
-    } catch (const std::system_error &) {  // no more threads: the rest here
-        std::memcpy(dst + at, src + at, bytes - at);
-    }
-    std::memcpy(dst, src, std::min(step, bytes));
-    for (auto &t : threads) t.join();
-}
 
 // Device memory to the caller's (pageable) memory through the pinned staging buffers, on the side stream: each piece's
 // copy to the host runs while the piece before it is copied on. 59 MB straight to pageable memory took 6 ms.
