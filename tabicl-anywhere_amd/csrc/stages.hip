@@ -428,13 +428,14 @@ __global__ __launch_bounds__(256) void k_rope(size_t rows, int T, int e, int hea
 }
 
 // ---- the class tokens' attention within each row: head width 16, at most 4 queries, T <= 64 J ---------------------
-// grid (n rows, heads / H); 64 x H threads (at most 8 heads), a wavefront a head. Few queries against the row's keys: plain
-// f32 arithmetic, each row's keys and values read once (the heads' slices of a token side by side). Rows of more than
-// 128 tokens take J = 4 with H = 4 heads a workgroup, whose LDS then still holds two workgroups a compute unit. Lane l
-// takes tokens l + 64 j: their keys (rotated, the k_rope formula) and values, the scores of the (rotated, 1 / sqrt(16))
-// queries, the softmax over the row's tokens by wavefront reductions; the weights and values then go through LDS,
-// and lane c = 16 i + j forms coordinate j of query i's output. Keys of token t of row r at kv + r * kv_row +
-// t * kv_tok (values e floats further), query i at q + r * q_row + i * q_tok.
+// grid (n rows, heads / H); 64 x H threads, a wavefront a head (the heads a multiple of H, so that every wavefront of a
+// workgroup reaches its barrier). Few queries against the row's keys: plain f32 arithmetic, each row's keys and values
+// read once (the heads' slices of a token side by side). Rows of more than 128 tokens take J = 4 with H = 4 heads a
+// workgroup, whose LDS then still holds two workgroups a compute unit. Lane l takes tokens l + 64 j: their keys (rotated,
+// the k_rope formula) and values, the scores of the (rotated, 1 / sqrt(16)) queries, the softmax over the row's tokens by
+// wavefront reductions; the weights and values then go through LDS, and lane c = 16 i + j forms coordinate j of query
+// i's output. Keys of token t of row r at kv + r * kv_row + t * kv_tok (values e floats further), query i at
+// q + r * q_row + i * q_tok.
 constexpr int CLS_MAXQ = 4;
 template <int J, int H>
 __global__ __launch_bounds__(64 * H) void k_cls_attn(int n, int T, int nq, int e, const float *__restrict__ kv,
@@ -444,7 +445,6 @@ __global__ __launch_bounds__(64 * H) void k_cls_attn(int n, int T, int nq, int e
     __shared__ float ps[H][CLS_MAXQ][64 * J];            // [head][query][token] weights
     __shared__ __align__(16) float vs[H][64 * J][16];    // [head][token][coordinate] values
     const int r = blockIdx.x, wave = threadIdx.x >> 6, h = blockIdx.y * H + wave, lane = threadIdx.x & 63;
-    if (h * 16 >= e) return;  // whole wavefronts leave together
     const float *kr = kv + (size_t)r * kv_row + h * 16;
     float k2[J][16];
     bool tl[J];
@@ -1060,6 +1060,12 @@ bool row_stage_takes_kv(const tah_weights *w, int n, int T) {
     return w->row_blocks >= 2 && row_block_path(w, 0, n, T) && row_kv_fits(w->row[0]);
 }
 
+// Whether k_cls_attn takes the last block's class tokens from cls_queries_min rows: eight heads fill its workgroups (the
+// weight image, of a block of width 128, and the head width of 16 leave no other count).
+static bool cls_kernel_fits(const tah_weights *w) {
+    return w->row[w->row_blocks - 1].inimg && w->cls <= CLS_MAXQ && w->row_heads == 8;
+}
+
 // Whether row_stage runs n rows of T tokens on the fused kernels alone: every block before the last as k_row_block
 // with its feed-forward half inside, the last through the class-token path and k_cls_attn. Its scratch is then
 // compact: the keys and values [n T][2 e] and the class tokens' buffers ([n cls] rows), not the per-token buffers of
@@ -1070,7 +1076,7 @@ static bool row_stage_compact(const tah_weights *w, int n, int T) {
     const size_t R = (size_t)n * T;
     for (int bi = 0; bi < last; bi++)
         if (!row_block_path(w, bi, n, T) || !block_ff_fits(w->row[bi]) || R <= SMALL_ROWS) return false;
-    return w->row[last].inimg && n >= cls_queries_min(T) && w->cls <= CLS_MAXQ && w->row_heads <= 8;
+    return cls_kernel_fits(w) && n >= cls_queries_min(T);
 }
 
 // The row stage's scratch, in floats; row_stage lays it out as:
@@ -1136,7 +1142,7 @@ void row_stage(hipStream_t s, const tah_weights *w, float *tok, int n, int T, co
     // the last block's path: only the class tokens queried (from cls_queries_min rows), by k_cls_attn where it
     // takes the shape
     const bool cls_path = fused && w->row[last].inimg && n >= cls_queries_min(T);
-    const bool cls_kernel = cls_path && cls <= CLS_MAXQ && heads <= 8;
+    const bool cls_kernel = cls_path && cls_kernel_fits(w);
     // kv_ready: this block's keys and values are in qkv [R][2 e] already (formed by the block before it)
     for (int bi = 0; bi <= last; bi++) {
         const DevBlock &b = w->row[bi];
@@ -1174,10 +1180,10 @@ void row_stage(hipStream_t s, const tah_weights *w, float *tok, int n, int T, co
             rows128(s, M, e, xc, e, b.inimg, b.ins, b.in_b, ac, e, EPI_NONE, nullptr, 0, nullptr, b.n1w, b.n1b);
             if (cls_kernel) {
                 if (T <= 128)
-                    hipLaunchKernelGGL((k_cls_attn<2, 8>), dim3(n), dim3(64 * heads), 0, s, n, T, cls, e, qkv,
+                    hipLaunchKernelGGL((k_cls_attn<2, 8>), dim3(n), dim3(512), 0, s, n, T, cls, e, qkv,
                                        (size_t)T * 2 * e, 2 * e, ac, (size_t)cls * e, e, cosv, sinv, att);
                 else
-                    hipLaunchKernelGGL((k_cls_attn<4, 4>), dim3(n, (heads + 3) / 4), dim3(256), 0, s, n, T, cls, e, qkv,
+                    hipLaunchKernelGGL((k_cls_attn<4, 4>), dim3(n, 2), dim3(256), 0, s, n, T, cls, e, qkv,
                                        (size_t)T * 2 * e, 2 * e, ac, (size_t)cls * e, e, cosv, sinv, att);
                 TAH_LAUNCHED();
             } else {
