@@ -265,9 +265,15 @@ static void launch_quantile_stats(hipStream_t s, int rows, int n, const float *q
     // as many rows a workgroup as leave four workgroups' LDS on a compute unit (at most the tails' 32), once there are
     // rows for two workgroups a compute unit of one row each
     constexpr int ROWS = K == 16 ? 8 : K == 8 ? 16 : 32;
-    const int per = std::min(ROWS, (rows + 511) / 512);
-    hipLaunchKernelGGL((k_quantile_stats<K, ROWS, 8>), dim3((rows + per - 1) / per), dim3(512), 0, s, rows, per, n, q, na,
-                       alphas, stats);
+    const int per = std::min(ROWS, rows / 512 + (rows % 512 > 0));
+    // at most 2^31 threads a launch (33 million rows of eight a workgroup)
+    const int most = per << 22;
+    for (int r0 = 0; r0 < rows;) {
+        const int here = std::min(most, rows - r0);
+        hipLaunchKernelGGL((k_quantile_stats<K, ROWS, 8>), dim3(here / per + (here % per > 0)), dim3(512), 0, s, here, per, n,
+                           q + (size_t)r0 * n, na, alphas, stats + (size_t)r0 * (3 + na));
+        r0 += here;
+    }
     TAH_LAUNCHED();
 }
 

@@ -8,7 +8,7 @@ import pytest
 from conftest import pkg
 from test_gpu_quantiles import host_stats, rows_of, say
 
-hip = pkg("hip")
+dm, hip = pkg("devmem"), pkg("hip")
 pytestmark = pytest.mark.gpu
 
 
@@ -41,3 +41,32 @@ def test_quantile_sizes(gpu, n, rows, levels):
     assert np.array_equal(np.isfinite(gt), ok)
     if ok.any():
         assert (np.abs(gt[ok] - wt[ok]) / np.maximum(np.abs(wt[ok]), 1.0)).max() < 5e-5
+
+
+def test_every_row_count(gpu):
+    """The largest row count there is, two quantiles a row (43 GB of quantiles and statistics on the card): a million rows
+    over and over, whose statistics come out alike everywhere, at the ends and wherever a launch could end."""
+    rows, period = 2 ** 31 - 1, 1 << 20
+    rng = np.random.default_rng(11)
+    part = rng.standard_normal((period, 2)).astype(np.float32)
+    want = gpu.quantile_stats(part, np.zeros(0, np.float32))
+    try:
+        q, out = dm.DeviceBuffer(rows * 8), dm.DeviceBuffer(rows * 12)
+    except RuntimeError:
+        pytest.skip("needs 43 GB of free memory on the card")
+    say(f"quantile sizes n=2 rows={rows}")
+    q.upload(part)
+    at = period
+    while at < rows:  # the rows so far once more behind themselves
+        n = min(at, rows - at)
+        assert dm.rt().hipMemcpy(q.ptr + 8 * at, q.ptr, 8 * n, 3) == 0
+        at += n
+    dm.synchronize()
+    gpu.quantile_stats_dev(q.ptr, rows, 2, np.zeros(0, np.float32), out.ptr)
+    got = np.empty((period, 3), np.float32)
+    for k in sorted({0, 2047} | set(range(127, 2048, 128)) | set(range(128, 2048, 128))):
+        n = min(period, rows - k * period)
+        assert dm.rt().hipMemcpy(got.ctypes.data, out.ptr + 12 * k * period, 12 * n, dm.D2H) == 0
+        assert np.array_equal(got[:n], want[:n]), k
+    q.free()
+    out.free()
