@@ -115,18 +115,22 @@ def query(block, scale: np.ndarray, x: np.ndarray) -> np.ndarray:
 
 def query_scales(blocks, n: int) -> np.ndarray:
     """`Block::query_scale` (`src/nn.rs:97-107`) of each block, [blocks][d]: what its queries are multiplied by with n
-    keys. The blocks' hidden units go through GELU together, and each row's sum runs left to right in float32, as the
-    reference's matvec rows: the products' columns as contiguous rows, summed row after row."""
+    keys. The blocks' hidden units go through GELU together (each block's own count of them, which may be none), and
+    each row's sum runs left to right in float32, as the reference's matvec rows: the products' columns as contiguous
+    rows, summed row after row."""
     out = np.empty((len(blocks), blocks[0].d), F)
-    inv = F(1.0) / np.sqrt(F(blocks[0].hd))
-    if blocks[0].ss_hidden == 0:
-        out[:] = inv
-        return out
     logn = np.log(F(max(n, 1)))
-    hid = gelu(np.stack([b.t["b0w"] for b in blocks]) * logn + np.stack([b.t["b0b"] for b in blocks]))
-    prod = np.empty((blocks[0].ss_hidden, blocks[0].d), F)
+    scaled = [b for b in blocks if b.ss_hidden]
+    if scaled:
+        hid = gelu(np.concatenate([b.t["b0w"] for b in scaled]) * logn + np.concatenate([b.t["b0b"] for b in scaled]))
+    at = 0
     for i, b in enumerate(blocks):
-        np.multiply(b.t["b2w"].reshape(b.d, b.ss_hidden).T, hid[i][:, None], out=prod)
+        inv = F(1.0) / np.sqrt(F(b.hd))
+        if b.ss_hidden == 0:
+            out[i] = inv
+            continue
+        prod = np.multiply(b.t["b2w"].reshape(b.d, b.ss_hidden).T, hid[at:at + b.ss_hidden, None], order="C")
+        at += b.ss_hidden
         np.add.reduce(prod, axis=0, dtype=F, out=out[i])
         out[i] = (out[i] + b.t["b2b"]) * inv
     return out

@@ -31,6 +31,28 @@ def test_query_scale_matches_the_oracle(tiny_model):
                 assert np.abs(got - want).max() <= 2e-7 * max(1.0, np.abs(want).max()), (n,)
 
 
+def test_query_scales_of_unlike_blocks():
+    """Each block's own hidden units and head width, summed left to right, whatever the others' are."""
+    rng = np.random.default_rng(3)
+    F, d, blocks = np.float32, 48, []
+    for heads, hid in ((4, 24), (3, 0), (6, 40), (4, 24), (2, 1)):
+        t = {"l1b": np.zeros(1, F)}
+        if hid:
+            t.update(b0w=rng.standard_normal(hid), b0b=rng.standard_normal(hid), b2w=rng.standard_normal(d * hid),
+                     b2b=rng.standard_normal(d))
+        blocks.append(M.Block(d, heads, t))
+    for n in (1, 777, 10000):
+        got = fit.query_scales(blocks, n)
+        for b, g in zip(blocks, got):
+            inv = F(1.0) / np.sqrt(F(b.hd))
+            want = np.full(d, inv, F)
+            if b.ss_hidden:
+                h = fit.gelu(b.t["b0w"] * np.log(F(n)) + b.t["b0b"])
+                s = np.add.accumulate(b.t["b2w"].reshape(d, -1) * h[None, :], axis=1, dtype=F)[:, -1]
+                want = (s + b.t["b2b"]) * inv
+            assert np.array_equal(g, want) and np.array_equal(fit.query_scale(b, n), want)
+
+
 def test_bundle_round_trip(tmp_path):
     t = {"a": np.arange(7, dtype=np.float32), "b": np.arange(6, dtype=np.int32).reshape(2, 3),
          "c": np.frombuffer(b"hello", dtype=np.uint8), "d": np.ones((2, 2), np.float16)}
