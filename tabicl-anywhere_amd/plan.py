@@ -37,7 +37,9 @@ class Plan:
 
     @classmethod
     def new(cls, max_classes: int, y, classes: int) -> "Plan":
-        y = np.asarray(y, np.float64).tolist()
+        # an array of numbers in one pass; whatever else float() takes, one by one
+        plain = isinstance(y, np.ndarray) and y.ndim == 1 and y.dtype.kind in "fiub"
+        y = y.astype(np.float64).tolist() if plain else [float(v) for v in y]
         mx = max_classes
         if mx == 0 or classes <= mx:
             return cls([max(classes, 1)], [Node(None, list(y), classes, True, list(range(classes)))])

@@ -3,6 +3,7 @@ its elementary functions (checked against the oracle, which is pinned to the ref
 import os
 
 import numpy as np
+import pytest
 
 import oracle as orc
 from conftest import GOLDEN, pkg
@@ -80,3 +81,25 @@ def test_copy_records_is_an_exact_copy():
         assert np.array_equal(got, src)
         if n:
             assert not np.shares_memory(got, src)
+
+
+@pytest.mark.filterwarnings("ignore:Conversion of an array")
+def test_plan_takes_any_sequence_of_numbers():
+    """Targets as an array, a column, a list, texts, a generator, or values that only float() reads."""
+    planmod = pkg("plan")
+
+    class Number:
+        def __init__(self, v):
+            self.v = v
+
+        def __float__(self):
+            return float(self.v)
+
+    values = [0, 3, 1, 12, 7, 5, 3, 11, 2, 4, 6, 8, 9, 10]
+    want = planmod.Plan.new(10, values, 13)
+    forms = [np.array(values, np.float32), np.array(values), np.array(values, object), np.array(values)[:, None],
+             [str(v) for v in values], [Number(v) for v in values]]
+    for y in forms:
+        assert planmod.Plan.new(10, y, 13) == want
+    assert planmod.Plan.new(10, (v for v in values), 13) == want
+    assert planmod.Plan.new(0, np.array([0.5, -2.25], np.float32), 5).nodes[0].y == [0.5, -2.25]
