@@ -1531,8 +1531,8 @@ __global__ __launch_bounds__(256, 1) void k_attn_few(int nq, int rows, int chunk
 // ---- split merge: Soft::merge then Soft::finish ---------------------------------------------------------------
 // grid nq * heads; 64 threads. The largest running maximum first (lanes over splits), then one pass over the
 // splits accumulating each one's weight sum and weighted values rescaled to it; loads are independent across
-// splits, so they stream. Maxima are in log2 units when log2_units is set, natural units otherwise.
-__global__ __launch_bounds__(64) void k_attn_merge(int nq, int d, int heads, int splits, int log2_units,
+// splits, so they stream. Maxima are in log2 units.
+__global__ __launch_bounds__(64) void k_attn_merge(int nq, int d, int heads, int splits,
                                                     const float *__restrict__ part_o,
                                                     const float *__restrict__ part_ml, float *__restrict__ out) {
     const int item = blockIdx.x, lane = threadIdx.x;
@@ -1551,8 +1551,7 @@ __global__ __launch_bounds__(64) void k_attn_merge(int nq, int d, int heads, int
         for (int s = 0; s < splits; s++) {
             const size_t at = s * stride + base;
             const float ls = part_ml[at * 2 + 1];
-            const float dm = part_ml[at * 2] - M;
-            const float f = ls > 0.0f ? (log2_units ? exp2_hw(dm) : fast_exp(dm)) : 0.0f;
+            const float f = ls > 0.0f ? exp2_hw(part_ml[at * 2] - M) : 0.0f;
             L += ls * f;
             O += part_o[at * hd + c] * f;
         }
@@ -1917,7 +1916,7 @@ void attention(hipStream_t s, const AttnShape &a, const float *q, const uint8_t 
             hipLaunchKernelGGL(k_attn_merge_w, dim3((a.nq * a.heads + 3) / 4), dim3(256), 0, s, a.nq * a.heads,
                                p.splits, part_o, part_ml, out);
         else
-            hipLaunchKernelGGL(k_attn_merge, dim3(a.nq * a.heads), dim3(64), 0, s, a.nq, a.d, a.heads, p.splits, 1,
+            hipLaunchKernelGGL(k_attn_merge, dim3(a.nq * a.heads), dim3(64), 0, s, a.nq, a.d, a.heads, p.splits,
                                part_o, part_ml, out);
         TAH_LAUNCHED();
     }
