@@ -207,8 +207,8 @@ int tah_fit_represent(tah_dev *dev, const tah_weights *w, const float *x, const 
 /* The fit hooks one at a time, with the trait's own layouts, for an unmodified fit_raw_async (src/fit.rs:425-545).
  *
  * Attend::column_batch (src/fit.rs:54, Gpu src/gpu.rs:1502-1510): how many feature groups of `rows` training cells
- * tah_columns takes per call within the working-memory budget left now; 0 when the column stage is not offered
- * (weights uploaded without the fitting blocks, or not even one group fits). */
+ * tah_columns takes per call, and any fewer, within the working-memory budget left now; 0 when the column stage is not
+ * offered (weights uploaded without the fitting blocks, or not even one group fits). */
 size_t tah_column_batch(const tah_dev *dev, const tah_weights *w, int32_t rows);
 /* Attend::columns (src/fit.rs:57, Gpu src/gpu.rs:1512-1614): the column stage for `groups` feature groups at once
  * (one label digit). cells [rows][groups][e] holds their training cells through the input layer with the target's
@@ -218,7 +218,7 @@ size_t tah_column_batch(const tah_dev *dev, const tah_weights *w, int32_t rows);
 int tah_columns(tah_dev *dev, const tah_weights *w, float *cells, int32_t rows, int32_t groups, const float *ind_q,
                 float *rec);
 /* Attend::row_batch (src/fit.rs:60, Gpu src/gpu.rs:1616-1622): how many rows of `features` cells tah_rows takes per
- * call; 0 when the row stage is not offered. */
+ * call, and any fewer; 0 when the row stage is not offered. */
 size_t tah_row_batch(const tah_dev *dev, const tah_weights *w, int32_t features);
 /* Attend::rows (src/fit.rs:63, Gpu src/gpu.rs:1624-1648): the row stage for n rows, cells [n][features][e] (after
  * the column stage) to reps [n][d]. */

@@ -459,8 +459,9 @@ __device__ __forceinline__ void in_cell8(const InCells &ic, const float (&vals)[
 //    two heads; behind these the rows of ones.
 // Matrix work and vector work take turns here: of a SIMD's cycles with two wavefronts 38% are matrix, 50% vector
 // instructions (1,000,000 cells without the input layer, 1.0 ms by counters). With a running maximum, its branches and the
-// head's projection inside the loop a wavefront issued 9,300 vector instructions for 32 cells, now 8,300; 102,400 cells
-// on one of two streams 252 -> 238 us, the 148 workgroups of 777 rows' halves 70 -> 61 us.
+// head's projection inside the loop a wavefront issued 9,300 vector instructions for 32 cells, now 8,340; 102,400 cells
+// on one of two streams 252 -> 238 us, the 148 workgroups of 777 rows' halves 70 -> 61 us. The queries' own scale a head
+// and the outputs' up to it, instead of one for all heads, are 40 of them (2,048 rows 3.70 -> 3.71 ms).
 // With FF the block's feed-forward half follows in the same kernel (ff128_rows, its weight slices in the same 64 KB
 // of LDS): the cells' new values stay in registers as its input; they are written out as well, for its residual add.
 // With KV as well the result goes on to the first row block's keys and values (ff128_rows with KV): cell (r, g)'s at

@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void k_col_records(int gb, int inds, int e, co
 // 16. A workgroup takes one group's head over a range of cells, wavefront w its inducing points 32 w .. of the 128 from
 // 128 (blockIdx.z) on: blocks of 128 cells are staged in LDS as split fp16 halves (one block ahead, each thread a key or
 // two coordinates of eight values), then attended as in the fused blocks (attend.hpp), the running maximum carried.
-// Bound by vector work (about ten instructions a score). All heads of a group run on the same XCD, one after another:
+// Bound by vector work (about ten instructions a score; of a SIMD's cycles 72% vector, 32% matrix). All heads of a group run on the same XCD, one after another:
 // a row's 2 e floats are read 64 bytes a head, and the heads share the lines in that XCD's L2. 100 groups of 10,000
 // cells: 518 us a launch, 1,090 on f32 MFMA with 64 cells a step and their loads waited for at each.
 constexpr int IND_NT = 128, IND_BUF = IND_NT * 128 + 2 * IND_NT * 32;  // a staged block and its rows of ones
@@ -429,7 +429,8 @@ void tokens_gmajor(hipStream_t s, const tah_weights *w, int rb, int r0, int rows
 }
 
 // Ranges of cells a group's head is split into, in blocks of 128: about 4,096 workgroups in all (768 run at once), at
-// least two blocks each.
+// least two blocks each. A launch with its merge, us, with 1,024, 2,048, 4,096 and 8,192 workgroups instead: 100 groups
+// of 10,000 cells 601, 522, 516, 518; 200 of 1,500 157, 158, 164, 162; 20 of 3,000 43, 46, 48, 46; 12 of 400 13 to 14.
 static int ind_splits(const tah_weights *w, int rows, int gb) {
     const int blocks = (rows + IND_NT - 1) / IND_NT;
     const int tiles = gb * w->col_heads * ((w->inds + 127) / 128);

@@ -31,7 +31,7 @@ namespace tah {
 // and values, all of them before its feed-forward half starts).
 //
 // W = 8 takes rows of 129 to 256 tokens, one workgroup a compute unit (two wavefronts a SIMD, as two workgroups of W =
-// 4). Measured with KV: 500 rows of 204 tokens 264 us a launch with the eight wavefronts (480 with the projection, the
+// 4). Measured with KV: 500 rows of 204 tokens 265 us a launch with the eight wavefronts (480 with the projection, the
 // rotation, the f32-MFMA attention, the output projection and the feed-forward apart). R = 2: 389 rows of 41 tokens 84
 // us as 389 workgroups, 64 us as 195.
 template <bool FF, bool KV, int W, int R, int NTL>

@@ -832,8 +832,11 @@ constexpr int SMALL_ROWS = 2048;
 // row 0.84 -> 0.76 ms a prediction, 64 rows 1.43 -> 1.40 ms).
 constexpr int ROW_BLOCK_MIN = 128;
 // The last row block queries the class tokens alone from this many rows: 512 of up to 128 tokens, every row count that
-// the row block takes of more, whose other tokens' queries cost more (204 tokens, a prediction without and with: 140
-// rows 0.981 and 0.970 ms, 200 1.033 and 0.996, 500 1.656 and 1.591).
+// the row block takes of more, whose other tokens' queries cost more. A prediction without and with, ms: rows of 204
+// tokens, 140 rows 0.981 and 0.970, 200 1.033 and 0.996, 500 1.656 and 1.591; of 104, 128 rows 0.760 and 0.760, 256
+// 0.810 and 0.801, 511 1.050 and 1.021; of 41, 128 rows 0.732 and 0.738, 256 0.768 and 0.767, 388 0.828 and 0.823, 511
+// 0.850 and 0.840; of 16, 192 rows 0.733 and 0.737, 511 0.825 and 0.818. At 512 the path pays at every width; below, it
+// loses up to 0.8% at 128 and 192 rows of few tokens and gains up to 2.8% from 256 rows of many.
 static int cls_queries_min(int T) { return T <= 128 ? 512 : ROW_BLOCK_MIN; }
 
 // x [M][e] += l2(gelu(l1(norm2 x))): the fused kernel where the block's shape has one (above SMALL_ROWS rows), else
@@ -1168,8 +1171,7 @@ void row_stage(hipStream_t s, const tah_weights *w, float *tok, int n, int T, co
             // the last block queries only the class tokens: keys and values for every token (the projection's second
             // and third 128-row blocks: qkv [R][2 e] for k_cls_attn, unless the previous block formed them, else into
             // qkv's [T][3 e] rows), queries for the class tokens alone, from their gathered copy (which the block
-            // then updates); below cls_queries_min rows the extra launch costs more than the other tokens' queries
-            // (2,048 rows 4.30 -> 4.25 ms, 64 and 256 rows 5 us slower)
+            // then updates)
             if (!kv_ready)
                 rows128(s, (int)R, 2 * e, tok, e, b.inimg + (size_t)128 * e * 4, b.ins, b.in_b + e,
                         cls_kernel ? qkv : qkv + e, cls_kernel ? 2 * e : 3 * e, EPI_NONE, nullptr, 0, nullptr, b.n1w,

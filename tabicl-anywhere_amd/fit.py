@@ -123,13 +123,15 @@ def query_scales(blocks, n: int) -> np.ndarray:
     scaled = [b for b in blocks if b.ss_hidden]
     if scaled:
         hid = gelu(np.concatenate([b.t["b0w"] for b in scaled]) * logn + np.concatenate([b.t["b0b"] for b in scaled]))
-    at = 0
+    at, prod = 0, np.empty((0, 0), F)
     for i, b in enumerate(blocks):
         inv = F(1.0) / np.sqrt(F(b.hd))
         if b.ss_hidden == 0:
             out[i] = inv
             continue
-        prod = np.multiply(b.t["b2w"].reshape(b.d, b.ss_hidden).T, hid[at:at + b.ss_hidden, None], order="C")
+        if prod.shape != (b.ss_hidden, b.d):
+            prod = np.empty((b.ss_hidden, b.d), F)
+        np.multiply(b.t["b2w"].reshape(b.d, b.ss_hidden).T, hid[at:at + b.ss_hidden, None], out=prod)
         at += b.ss_hidden
         np.add.reduce(prod, axis=0, dtype=F, out=out[i])
         out[i] = (out[i] + b.t["b2b"]) * inv
