@@ -1,4 +1,4 @@
-"""Heads of very different magnitude in the fused column and row blocks: one head's numbers are 2^30 times the others' and
+"""Heads of very different magnitude in the fused column and row blocks and the inducing points' attention: one head's numbers are 2^30 times the others' and
 have no part in the result, so that the other heads must come out as if it were not there. Against the oracle at the
 stages' raw-score tolerance, 5e-5; a scale shared with the large head would leave the others eight bits.
 
@@ -26,7 +26,7 @@ def gpu():
 
 def large_queries():
     m = M.Model.random(M.FULL_CLASSIFIER, seed=2)
-    for b in m.col_a2 + m.row[:-1]:
+    for b in m.col_a1 + m.col_a2 + m.row[:-1]:
         e = b.d
         b.t["in_b"][:16] = BIG
         b.t["in_w"].reshape(3 * e, e)[e:e + 16] = 0.0
@@ -36,7 +36,7 @@ def large_queries():
 
 def large_values():
     m = M.Model.random(M.FULL_CLASSIFIER, seed=2)
-    for b in m.col_a2 + m.row[:-1]:
+    for b in m.col_a1 + m.col_a2 + m.row[:-1]:
         e = b.d
         b.t["in_b"][2 * e + 112:] = BIG
         b.t["out_w"].reshape(e, e)[:, 112:] = 0.0
@@ -96,3 +96,21 @@ def test_fit_columns(gpu, kind, model, weights):
     err = max(np.abs(got - want)[keep].max(), np.abs(reps - orc.fit_rows(model, emb)).max())
     say(f"large {kind}, a fit: {err:.2e}")
     assert err < TOL
+
+
+@pytest.mark.parametrize("place", [0, 350, 699])
+def test_outlying_cell(gpu, place):
+    """A row a million times the others', first, within and last of the inducing points' ranges of cells: the scale that
+    their keys and values take from it must not cost the others, nor depend on where it stands."""
+    m = M.Model.random(M.FULL_CLASSIFIER, seed=2)
+    w = gpu.weights(m)
+    rng = np.random.default_rng(9)
+    x, y = rng.standard_normal((700, 3)).astype(np.float32), rng.integers(0, 10, 700).astype(np.float32)
+    x[place] *= 1e6
+    got, reps = gpu.fit_represent(w, x, y, [10], np.stack([fit.query_scale(b, 700) for b in m.col_a1]))
+    want, emb = orc.fit_columns(m, x, y, [10], 256)
+    # head by head, each against its own size
+    g, t = (a.reshape(3, 3, 2, 8, 16, m.inds) for a in (got, want))
+    off = np.abs(g - t).max(axis=(0, 4, 5)) / np.abs(t).max(axis=(0, 4, 5))
+    say(f"an outlying cell at {place}: {off.max():.2e} of a head, rows {np.abs(reps - orc.fit_rows(m, emb)).max():.2e}")
+    assert off.max() < TOL and np.abs(reps - orc.fit_rows(m, emb)).max() < TOL
